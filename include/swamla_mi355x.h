@@ -398,6 +398,53 @@ int mla_head_product(const void* x, int64_t x_rs, int64_t x_hs,
                      int64_t y_rs, int64_t y_hs, int32_t M, int32_t N,
                      int32_t K, int32_t H, int32_t dtype, void* stream);
 
+/*
+ * mla_head_product_rows — the per-head product of rows that every head
+ * shares, batch by batch: y[b][h][m][n] = sum_k x[b][m][k] * w[h][n][k], fp32
+ * accumulation, one rounding to bf16.  Replaces the up-projection of cached
+ * latents into a head's keys and values (models/mla.py:427-437): x = cache
+ * rows (row stride x_rs, sequence stride x_bs), w = W_uk or W_uv [H, 128,
+ * R_pad].  x_dtype bf16, or e4m3 codes with one fp32 scale per row (x_scale
+ * + b*scale_bs + m; the sum is scaled before the rounding).  y: row y_rs,
+ * head y_hs, sequence y_bs; n contiguous.
+ * Limits: K a multiple of 64 up to 1024, N a multiple of 64, H*N <= 2^22; x
+ * and w 16-byte aligned with strides of whole 16 bytes, y 8-byte aligned with
+ * strides that are multiples of 4.
+ */
+int mla_head_product_rows(const void* x, int64_t x_rs, int64_t x_bs,
+                          const float* x_scale, int64_t scale_bs,
+                          const void* w, int64_t w_rs, int64_t w_hs, void* y,
+                          int64_t y_rs, int64_t y_hs, int64_t y_bs, int32_t B,
+                          int32_t M, int32_t N, int32_t K, int32_t H,
+                          int32_t x_dtype, void* stream);
+
+/*
+ * mla_prompt_attn — causal attention of T new tokens per sequence, all from
+ * position start, over expanded keys and values (models/mla.py:427-487 as the
+ * reference computes it; the counterpart of mla_prefill_attn, which carries
+ * the queries through the latent space): token t of sequence b attends to
+ * [0, start + t].
+ *   s = sm_scale * (q_nope . k + rope(q_pe) . k_pe),  out = softmax(s) v
+ * q            token r = b*T + t, head h at q + r*q_rs + h*q_hs: 128 nope
+ *              channels, then 64 rope channels (unrotated: rotated here by
+ *              table row t, or start + t with rope_abs).
+ * k, v         [B][H][start + T][128] contiguous (mla_head_product_rows); v
+ *              row positions 32c + 8a + 4f + e hold channel 64f + 16c + 4a + e
+ *              (the rows of its W_uv in that order).
+ * kpe_cache    [cache_batch][cache_seq][64].
+ * out          token r, head h at out + r*o_rs + h*o_hs, 128 values.
+ * bf16 only, nope 128, rope 64, v 128; bases 16-byte aligned, strides
+ * multiples of 8.
+ */
+int mla_prompt_attn(const void* q, int64_t q_rs, int64_t q_hs,
+                    const void* cos_tab, const void* sin_tab,
+                    int64_t rope_len, const void* k, const void* v,
+                    const void* kpe_cache, int64_t cache_batch,
+                    int64_t cache_seq, int32_t B, int32_t T, int32_t start,
+                    int32_t rope_abs, int32_t H, int32_t Dn, int32_t P,
+                    int32_t Dv, float sm_scale, void* out, int64_t o_rs,
+                    int64_t o_hs, int32_t dtype, void* stream);
+
 /* Split plan used by both kernels, exported so hosts and tests can size the
  * partial buffers: number of splits of a row of length L (0 for L <= 0). */
 int32_t mla_split_count(int32_t L, int32_t n_splits, int32_t min_chunk);

@@ -18,6 +18,7 @@ SOURCES = [
     os.path.join(HERE, "csrc", "mla_prefill.hip"),
     os.path.join(HERE, "csrc", "mla_linear.hip"),
     os.path.join(HERE, "csrc", "mla_absorb.hip"),
+    os.path.join(HERE, "csrc", "mla_prompt.hip"),
     os.path.join(HERE, "csrc", "mla_scratch.hip"),
     os.path.join(HERE, "csrc", "mla_probe.hip"),
     os.path.join(HERE, "csrc", "mla_abi.cpp"),
@@ -35,9 +36,13 @@ def hipcc() -> str:
 
 # Per-source options.  The decode kernel keeps its MFMA accumulators in
 # ordinary VGPRs (its softmax rescales them on the VALU every sub-tile, and
-# AGPR accumulators would be copied back and forth each time).
+# AGPR accumulators would be copied back and forth each time).  So do the
+# prompt pass's attention and products (at most 256 registers per wave, all
+# of them addressable as VGPRs).
 EXTRA = {
     "mla_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "mla_prompt.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "mla_absorb.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 BUILD_DIR = os.path.join(HERE, "_build")
 

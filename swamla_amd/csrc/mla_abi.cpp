@@ -586,9 +586,76 @@ int mla_head_product(const void* x, int64_t x_rs, int64_t x_hs, const void* w, i
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&n_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cus < 1)
     return hip_fail(fn);
-  swamla::HeadProductArgs a{x, x_rs, x_hs, w, w_rs, w_hs, y, y_rs, y_hs, M, N, K};
-  const int rc = swamla::launch_head_product(a, H, n_cus, static_cast<hipStream_t>(stream));
+  swamla::HeadProductArgs a{x, x_rs, x_hs, 0, nullptr, 0, w, w_rs, w_hs, y, y_rs, y_hs, 0, M, N, K, 1, H};
+  const int rc = swamla::launch_head_product(a, n_cus, static_cast<hipStream_t>(stream));
   if (rc == -1) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: no kernel for K=%d", fn, K);
+  if (rc != 0) return hip_fail(fn);
+  return ok();
+}
+
+int mla_head_product_rows(const void* x, int64_t x_rs, int64_t x_bs, const float* x_scale, int64_t scale_bs,
+                          const void* w, int64_t w_rs, int64_t w_hs, void* y, int64_t y_rs, int64_t y_hs,
+                          int64_t y_bs, int32_t B, int32_t M, int32_t N, int32_t K, int32_t H, int32_t x_dtype,
+                          void* stream) {
+  const char* fn = "mla_head_product_rows";
+  const bool fp8 = x_dtype == SWAMLA_DTYPE_FP8;
+  if (x_dtype != SWAMLA_DTYPE_BF16 && !fp8)
+    return fail(SWAMLA_ERR_UNSUPPORTED, "%s: x dtype %d not built (bf16 or e4m3)", fn, x_dtype);
+  if (B < 0 || M < 0 || N < 0 || H < 0 || static_cast<int64_t>(H) * N > (int64_t(1) << 22))
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: B=%d M=%d N=%d H=%d out of range", fn, B, M, N, H);
+  if (K < 64 || K > 1024 || K % 64 != 0)
+    return fail(SWAMLA_ERR_UNSUPPORTED, "%s: K=%d (built: multiples of 64 up to 1024)", fn, K);
+  if (N % 64 != 0) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: N=%d is not a multiple of 64", fn, N);
+  if (B == 0 || M == 0 || N == 0 || H == 0) return ok();
+  if (!x || !w || !y || fp8 != (x_scale != nullptr))
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: null x / w / y, or row scales without e4m3 rows (or the reverse)", fn);
+  if (x_rs < K || x_bs < 0 || scale_bs < 0 || w_hs < 0 || w_rs < K || y_rs < 0 || y_hs < 0 || y_bs < 0)
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: negative strides, or an x or w row stride below K", fn);
+  if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 8) || (x_scale && !aligned(x_scale, 4)) ||
+      (x_rs | x_bs) % (fp8 ? 16 : 8) != 0 || (w_rs | w_hs) % 8 != 0 || (y_rs | y_hs | y_bs) % 4 != 0)
+    return fail(SWAMLA_ERR_MISALIGNED, "%s: x and w need 16-byte aligned bases and strides of whole 16 bytes, y an "
+                "8-byte aligned base and strides that are multiples of 4", fn);
+  int dev = 0, n_cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cus < 1)
+    return hip_fail(fn);
+  swamla::HeadProductArgs a{x, x_rs, 0, x_bs, x_scale, scale_bs, w, w_rs, w_hs, y, y_rs, y_hs, y_bs, M, N, K, B, H};
+  const int rc = swamla::launch_head_product(a, n_cus, static_cast<hipStream_t>(stream));
+  if (rc == -1) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: no kernel for B=%d M=%d K=%d", fn, B, M, K);
+  if (rc != 0) return hip_fail(fn);
+  return ok();
+}
+
+int mla_prompt_attn(const void* q, int64_t q_rs, int64_t q_hs, const void* cos_tab, const void* sin_tab,
+                    int64_t rope_len, const void* k, const void* v, const void* kpe_cache, int64_t cache_batch,
+                    int64_t cache_seq, int32_t B, int32_t T, int32_t start, int32_t rope_abs, int32_t H, int32_t Dn,
+                    int32_t P, int32_t Dv, float sm_scale, void* out, int64_t o_rs, int64_t o_hs, int32_t dtype,
+                    void* stream) {
+  const char* fn = "mla_prompt_attn";
+  if (dtype != SWAMLA_DTYPE_BF16) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: dtype %d not built (bf16 only)", fn, dtype);
+  if (Dn != 128 || P != 64 || Dv != 128)
+    return fail(SWAMLA_ERR_UNSUPPORTED, "%s: nope %d, rope %d, v %d (built: 128, 64, 128)", fn, Dn, P, Dv);
+  if (B < 0 || T < 0 || H < 0 || start < 0)
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: B=%d T=%d H=%d start=%d out of range", fn, B, T, H, start);
+  if (B == 0 || T == 0 || H == 0) return ok();
+  if (!q || !cos_tab || !sin_tab || !k || !v || !kpe_cache || !out)
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: null pointer", fn);
+  if (cache_batch < B || static_cast<int64_t>(start) + T > cache_seq || cache_seq > (int64_t(1) << 31) - 1)
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: %d sequences of %d + %d tokens in a cache of %lld x %lld", fn, B, start, T,
+                (long long)cache_batch, (long long)cache_seq);
+  if (static_cast<int64_t>(B) * H > (int64_t(1) << 24))
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: B=%d x H=%d out of range", fn, B, H);
+  if (rope_len < 1 || !(sm_scale > 0.f)) return fail(SWAMLA_ERR_INVALID_ARG, "%s: bad RoPE table or scale", fn);
+  if (q_rs < 0 || q_hs < 192 || o_rs < 0 || o_hs < 128)
+    return fail(SWAMLA_ERR_INVALID_ARG, "%s: negative row strides, or head strides below 192 (q) / 128 (out)", fn);
+  if (!aligned(q, 16) || !aligned(cos_tab, 8) || !aligned(sin_tab, 8) || !aligned(k, 16) || !aligned(v, 16) ||
+      !aligned(kpe_cache, 16) || !aligned(out, 16) || (q_rs | q_hs | o_rs | o_hs) % 8 != 0)
+    return fail(SWAMLA_ERR_MISALIGNED, "%s: 16-byte aligned bases and strides that are multiples of 8 required", fn);
+  const float log2e = 1.4426950408889634f;
+  swamla::PromptArgs a{q, q_rs, q_hs, cos_tab, sin_tab, rope_len, k, v, kpe_cache, cache_seq * 64,
+                       B, H, T, start, rope_abs, sm_scale * log2e, out, o_rs, o_hs};
+  const int rc = swamla::launch_prompt(a, static_cast<hipStream_t>(stream));
+  if (rc == -1) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: too many query groups", fn);
   if (rc != 0) return hip_fail(fn);
   return ok();
 }

@@ -160,16 +160,40 @@ struct PackWeightArgs {
   int N, K;
 };
 
-// Per-head product of the prompt pass: y[m, h, n] = sum_k x[m, h, k] w[h, n, k]
-// (strides in elements; m < M, n < N, k < K).
+// Per-head product of the prompt pass: y[b, m, h, n] = sum_k x[b, m, h, k]
+// w[h, n, k] (strides in elements; b < B, m < M, n < N, k < K).  x_hs == 0: x
+// is the same for every head.  x_scale: x holds e4m3
+// codes, row (b, m) scaled by x_scale[b * s_bs + m] (x_hs == 0 and N % 64 == 0).
 struct HeadProductArgs {
   const void* x;
-  int64_t x_rs, x_hs;
+  int64_t x_rs, x_hs, x_bs;
+  const float* x_scale;
+  int64_t s_bs;
   const void* w;
   int64_t w_rs, w_hs;
   void* y;
-  int64_t y_rs, y_hs;
-  int M, N, K;
+  int64_t y_rs, y_hs, y_bs;
+  int M, N, K, B, H;
+  int shared = 0, y_wide = 0;  // set by the launcher: x_hs == 0 columns run over all heads; 16-byte stores
+};
+
+// Causal attention of a prompt over expanded keys and values (mla_prompt.hip):
+// token t of sequence b, of T from position start, attends to [0, start + t].
+struct PromptArgs {
+  const void* q;  // [B * T, H, 192]: 128 nope channels, then 64 rope channels (unrotated)
+  int64_t q_rs, q_hs;
+  const void* cos_tab;
+  const void* sin_tab;
+  int64_t rope_len;
+  const void* k;  // [B, H, start + T, 128]
+  const void* v;  // [B, H, start + T, 128], position 32 cb + 8 a + 4 f + e holding channel 64 f + 16 cb + 4 a + e
+  const void* kpe;  // sequence b's rows at b * kpe_bs elements, 64 each
+  int64_t kpe_bs;
+  int B, H, T, start;
+  int rope_abs;
+  float scale_log2;  // softmax_scale * log2(e)
+  void* out;  // [B * T, H, 128]
+  int64_t o_rs, o_hs;
 };
 
 // Measurement kernels (bench.py's roofline ceiling legs): a decode launch's
@@ -182,7 +206,8 @@ int launch_linear(const LinearArgs& a, int batch, hipStream_t s);
 int launch_linear_packed(const PackedLinearArgs& a, hipStream_t s);
 int launch_pack_weight(const PackWeightArgs& a, hipStream_t s);
 int launch_merge_project(const MergeProjectArgs& a, hipStream_t s);
+int launch_prompt(const PromptArgs& a, hipStream_t s);
 // -1: no kernel for this K; -2: launch error.
-int launch_head_product(const HeadProductArgs& a, int H, int n_cus, hipStream_t s);
+int launch_head_product(const HeadProductArgs& a, int n_cus, hipStream_t s);
 
 }  // namespace swamla

@@ -1,0 +1,300 @@
+// mla_prompt.hip — causal attention of a prompt over per-head keys and values
+// (the "expanded" association of models/mla.py:427-487).
+//
+// A prompt's queries each attend to about as many tokens as there are
+// queries, so it pays to expand every cached latent once into its heads' keys
+// and values (mla_head_product_rows: K = c W_uk^T, V = c W_uv^T), as the
+// reference does, instead of carrying queries and outputs through the latent
+// space: 2 (192 + 128) flops per head and (query, key) pair instead of
+// 2 (2 R_pad + 64), whatever the rank, and the keys need no per-token scale.
+//
+//   s = scale (q_nope . K[h, key] + rope(q_pe) . k_pe[key]),  o = softmax(s) V
+//
+// bf16 operands, fp32 scores, softmax and accumulation, bf16 softmax weights
+// (the sum is of the rounded weights), as the latent-space kernels do.
+//
+// Bound: MFMA, and nearly as much LDS: a wave's 40 MFMAs of a tile (32 cycles
+// each) read 40 KB of operands, 1 KB per MFMA.
+//
+// Schedule.  A workgroup of four waves takes 128 consecutive queries of one
+// (sequence, head), 32 per wave (the MFMA columns), and walks the 64-token
+// tiles of the causal range.  Two workgroups per CU (80 KB of LDS and at most
+// 256 registers per wave each), so that one's softmax and waits overlap the
+// other's MFMAs.
+//   S^T[32 tok x 32 q] = K Q^T   mfma_f32_32x32x16_bf16, A = K rows from LDS,
+//                                B = Q^T in registers for the whole walk
+//   O^T[32 ch x 32 q] += V^T P^T A = V read transposed (ds_read_b64_tr_b16);
+//                                the score registers' lane layout is the B
+//                                operand once the k slots of a 16-token step
+//                                are taken as tokens {4h .. 4h+3, 8+4h ..}
+// Tiles arrive by LDS copies (1 KB per instruction).  Keys run one tile ahead
+// of values: iteration j multiplies tile j + 1's QK and tile j's PV, so K and
+// V each need two buffers only: at iteration j's barrier, K buffer j % 2 and V
+// buffer (j + 1) % 2 are free and take K tile j + 2 and V tile j + 1.
+// LDS rows are 256 bytes (128 channels; k_pe rows 128 bytes), 16-byte chunk c
+// of row t at c ^ (((t & 3) << 2) | ((t >> 2) & 3)) (k_pe: c ^ ((t >> 1) & 7)):
+// both operand reads hit distinct banks.
+// The heaviest query groups (the last ones) are launched first, over all
+// (sequence, head) pairs in turn: with a multiple of 8 pairs each pair's
+// workgroups land on one XCD and stream its keys through one L2.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "mla_args.h"
+#include "mla_device.h"
+#include "mla_stream.h"
+#include "numerics.h"
+
+namespace swamla {
+namespace {
+
+constexpr int kPrWaves = 4;
+constexpr int kPrQ = 32 * kPrWaves;  // queries per workgroup
+constexpr int kPrTok = 64;           // tokens per tile
+constexpr int kPrD = 128;            // nope and value dimensions
+constexpr int kPrRow = 2 * kPrD;     // bytes per K / V row
+constexpr int kPrPe = 2 * kP;        // bytes per rope row
+constexpr int kPrKBytes = kPrTok * (kPrRow + kPrPe), kPrVBytes = kPrTok * kPrRow;
+
+__device__ __forceinline__ int pr_swz(int t) { return ((t & 3) << 2) | ((t >> 2) & 3); }
+
+__global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * (kPrKBytes + kPrVBytes)];
+  const uint32_t lds_k = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)lds));
+  const uint32_t lds_v = lds_k + 2 * kPrKBytes;
+
+  const int BH = a.B * a.H;
+  const int n_qb = (a.T + kPrQ - 1) / kPrQ;
+  const int qb_i = n_qb - 1 - static_cast<int>(blockIdx.x) / BH, bh = static_cast<int>(blockIdx.x) % BH;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 31, hf = lane >> 5;  // column (query), lane half
+  const int L = a.start + a.T;
+
+  const int t_w = qb_i * kPrQ + 32 * w;              // the wave's first query
+  const int t_end = min((qb_i + 1) * kPrQ, a.T);      // one past the block's last
+  const int tq = min(t_w + n, a.T - 1);               // surplus columns repeat the last query
+  const int Lq = a.start + tq + 1;                    // causal end of this column
+  const int Lw = a.start + min(t_w + 32, a.T);        // causal end of the wave's last query
+  const int n_tiles = (a.start + t_end + kPrTok - 1) / kPrTok;  // block-uniform, >= 1
+  // tiles this wave multiplies (a wave past the last query: none)
+  const int w_tiles = t_w < a.T ? (Lw + kPrTok - 1) / kPrTok : 0;
+
+  const uint8_t* const kb = static_cast<const uint8_t*>(a.k) + static_cast<int64_t>(bh) * L * kPrRow;
+  const uint8_t* const vb = static_cast<const uint8_t*>(a.v) + static_cast<int64_t>(bh) * L * kPrRow;
+  const uint8_t* const pe = static_cast<const uint8_t*>(a.kpe) + static_cast<int64_t>(b) * a.kpe_bs * 2;
+
+  // ---- tile copies: this wave's 16 rows (16 w ..).  K / V: 4 rows per copy,
+  // lane -> row 4 q + lane / 16, slot lane % 16; rope: 8 rows per copy.
+  const int cr = lane >> 4;
+  const uint32_t c0 = (lane & 15) ^ (cr << 2);  // chunk of copy q: c0 ^ q (pr_swz of row 4 q + cr is 4 cr + q)
+  auto copy_rows = [&](const uint8_t* base, int j, uint32_t dst) __attribute__((always_inline)) {
+    const int left = L - 1 - j * kPrTok;  // rows past the last re-read it
+    const uint8_t* const src = base + static_cast<int64_t>(j) * kPrTok * kPrRow;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = min(16 * w + 4 * q + cr, left);
+      st_copy16(dst + (16 * w + 4 * q) * kPrRow, r * kPrRow + 16 * (c0 ^ q), src);
+    }
+  };
+  auto copy_k = [&](int j) __attribute__((always_inline)) {
+    const uint32_t dst = lds_k + (j & 1) * kPrKBytes;
+    copy_rows(kb, j, dst);
+    const int left = L - 1 - j * kPrTok;
+    const uint8_t* const src = pe + static_cast<int64_t>(j) * kPrTok * kPrPe;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int r = 16 * w + 8 * q + (lane >> 3);
+      const uint32_t c = (lane & 7) ^ ((r >> 1) & 7);
+      st_copy16(dst + kPrTok * kPrRow + (16 * w + 8 * q) * kPrPe, min(r, left) * kPrPe + 16 * c, src);
+    }
+  };
+  auto copy_v = [&](int j) __attribute__((always_inline)) { copy_rows(vb, j, lds_v + (j & 1) * kPrVBytes); };
+
+  copy_k(0);
+  copy_v(0);
+  if (n_tiles > 1) copy_k(1);
+
+  // ---- Q^T operands: lane (n, hf) holds channels 16 ks + 8 hf .. + 7 of its
+  // query; k-steps 8 .. 11 are the rope part, rotated here (per-op rounding).
+  bf16x8_t qv[12];
+  {
+    const uint16_t* const qp =
+        static_cast<const uint16_t*>(a.q) + (static_cast<int64_t>(b) * a.T + tq) * a.q_rs + h * a.q_hs + 8 * hf;
+    uint4 raw[12];
+#pragma unroll
+    for (int ks = 0; ks < 12; ++ks) raw[ks] = *reinterpret_cast<const uint4*>(qp + 16 * ks);
+    int rp = a.rope_abs ? a.start + tq : tq;
+    rp = rp >= a.rope_len ? static_cast<int>(a.rope_len) - 1 : rp;
+    const uint16_t* const ct = static_cast<const uint16_t*>(a.cos_tab) + static_cast<int64_t>(rp) * (kP / 2) + 4 * hf;
+    const uint16_t* const st = static_cast<const uint16_t*>(a.sin_tab) + static_cast<int64_t>(rp) * (kP / 2) + 4 * hf;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qv[ks] = as_bf16x8(raw[ks]);
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+      const uint2 c2 = *reinterpret_cast<const uint2*>(ct + 8 * s4), s2 = *reinterpret_cast<const uint2*>(st + 8 * s4);
+      const uint32_t in[4] = {raw[8 + s4].x, raw[8 + s4].y, raw[8 + s4].z, raw[8 + s4].w};
+      uint32_t o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t cw = e < 2 ? c2.x : c2.y, sw = e < 2 ? s2.x : s2.y;
+        const uint32_t cj = (e & 1) ? cw >> 16 : cw & 0xFFFF, sj = (e & 1) ? sw >> 16 : sw & 0xFFFF;
+        o[e] = rope_bf16_packed(bf16_to_f32(in[e] & 0xFFFF), bf16_to_f32(in[e] >> 16), bf16_to_f32(cj),
+                                bf16_to_f32(sj));
+      }
+      qv[8 + s4] = as_bf16x8(make_uint4(o[0], o[1], o[2], o[3]));
+    }
+  }
+
+  f32x16_t oacc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) oacc[i] = f32x16_t{};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  // ---- operand addresses within a buffer (the swizzle XORs low chunk bits)
+  const uint32_t ko = n * kPrRow + 16 * (hf ^ pr_swz(n & 15));                        // ^ 32 ks, + 32 h2 rows
+  const uint32_t po = kPrTok * kPrRow + n * kPrPe + 16 * (hf ^ ((n >> 1) & 7));       // ^ 32 s
+  const int jj = lane & 15;
+  const int r0 = 4 * hf + (jj >> 2);  // row of the first transposed read; the second is 8 rows on, chunk ^ 2
+  const uint32_t to = r0 * kPrRow + 16 * ((2 * ((lane >> 4) & 1) + ((jj & 3) >> 1)) ^ pr_swz(r0)) + 8 * (jj & 1);
+
+  f32x16_t sc[2];
+  bf16x8_t pb[4];
+  const bf16x2_t ones = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
+
+  // LDS reads of the QK slots (one each) and the PV slots (two each) of an
+  // iteration form one stream, kAhead reads in flight.
+  constexpr int kQk = 24, kPv = 16, kAhead = 8;
+  // One stream of MFMAs: QK of the tile in K buffer kbuf (if QK), then PV of
+  // the tile in V buffer vbuf (if PV).
+  auto stream = [&](auto do_qk, auto do_pv, uint32_t kbuf, uint32_t vbuf) __attribute__((always_inline)) {
+    constexpr bool QK = decltype(do_qk)::value, PV = decltype(do_pv)::value;
+    constexpr int nq = QK ? kQk : 0, np = PV ? kPv : 0, reads = nq + 2 * np;
+    st_u32x4_t kr[QK ? kQk : 1];
+    s16x4_t vr[PV ? kPv : 1][2];
+    auto rd = [&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i < nq) {
+        constexpr int ks = i / 2, h2 = i % 2;
+        if constexpr (ks < 8) kr[i] = st_read<st_u32x4_t>(kbuf + (ko ^ (32 * ks)) + 32 * h2 * kPrRow);
+        else kr[i] = st_read<st_u32x4_t>(kbuf + (po ^ (32 * (ks - 8))) + 32 * h2 * kPrPe);
+      } else {
+        constexpr int m = (i - nq) / 2, e = (i - nq) % 2, s4 = m / 4, cb = m % 4;
+        vr[m][e] = st_read_tr(vbuf + (to ^ (64 * cb + 32 * e)) + (16 * s4 + 8 * e) * kPrRow);
+      }
+    };
+    if constexpr (QK) sc[0] = f32x16_t{}, sc[1] = f32x16_t{};
+    st_for<0, st_min(kAhead, reads)>(rd);
+    st_for<0, nq + np>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      constexpr int prev = i < nq ? i : nq + 2 * (i - nq);                // reads used by earlier slots
+      constexpr int done = i < nq ? i + 1 : nq + 2 * (i - nq + 1);         // by this one too
+      st_for<st_min(prev + kAhead, reads), st_min(done + kAhead, reads)>(rd);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (i < nq) {
+        constexpr int ks = i / 2, h2 = i % 2;
+        sc[h2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kr[i]), qv[ks], sc[h2], 0, 0, 0);
+      } else {
+        constexpr int m = i - nq, s4 = m / 4, cb = m % 4;
+        oacc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cat_bf16x8(vr[m][0], vr[m][1]), pb[s4], oacc[cb], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  // The online-softmax step of tile j's scores (after the PV of the tile
+  // before it): the reference moves lazily, per column, when its maximum
+  // grew by more than 2^kLazy; O is rescaled then.
+  auto softmax = [&](int j) __attribute__((always_inline)) {
+    if ((j + 1) * kPrTok > a.start + t_w + 1) {  // uniform: the tile reaches past the wave's first causal end
+      const int tok0 = j * kPrTok + 4 * hf;
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (tok0 + 32 * h2 + 8 * (r >> 2) + (r & 3) >= Lq) sc[h2][r] = -INFINITY;
+    }
+    float mt = sc[0][0];
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sc[h2][r]);
+    const auto r32 = __builtin_amdgcn_permlane32_swap(f2u(mt), f2u(mt), false, false);
+    mt = fmaxf(u2f(r32[0]), u2f(r32[1])) * a.scale_log2;
+    const bool mine = mt > m_run + kLazy;
+    const float m_new = mine ? mt : m_run;
+    if (__any(mine)) {
+      const float alpha = m_new == m_run ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);  // both -inf: 1, not NaN
+      l_run *= alpha;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) oacc[i] *= alpha;
+    }
+    m_run = m_new;
+    const float mref = m_new == -INFINITY ? 0.f : -m_new;
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb) {
+        uint32_t pw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[h2][8 * sb + 2 * e], a.scale_log2, mref));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[h2][8 * sb + 2 * e + 1], a.scale_log2, mref));
+          pw[e] = pack_bf16x2(p0, p1);
+          l_run = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pw[e]), ones, l_run, false);
+        }
+        pb[2 * h2 + sb] = as_bf16x8(make_uint4(pw[0], pw[1], pw[2], pw[3]));
+      }
+  };
+
+  using Y = std::true_type;
+  using N = std::false_type;
+  st_tile_barrier();
+  if (w_tiles > 0) {
+    stream(Y{}, N{}, lds_k, 0);
+    softmax(0);
+  }
+  for (int j = 0; j < n_tiles; ++j) {
+    st_tile_barrier();  // K tile j + 1 and V tile j complete; K tile j and V tile j - 1 consumed
+    if (j + 2 < n_tiles) copy_k(j + 2);
+    if (j + 1 < n_tiles) copy_v(j + 1);
+    const uint32_t kbuf = lds_k + ((j + 1) & 1) * kPrKBytes, vbuf = lds_v + (j & 1) * kPrVBytes;
+    if (j + 1 < w_tiles) {
+      stream(Y{}, Y{}, kbuf, vbuf);
+      softmax(j + 1);
+    } else if (j < w_tiles) {
+      stream(N{}, Y{}, 0, vbuf);
+    }
+  }
+  if (t_w + n >= a.T) return;  // surplus columns
+
+  // Lane (n, hf) holds positions 32 cb + 8 r4 + 4 hf + e of its query's
+  // output; V's rows are laid out so that these are channels
+  // 64 hf + 16 cb + 4 r4 + e: 128 contiguous bytes per lane.
+  const float l_w = l_run + shfl_xor_f32(l_run, 32);
+  const float inv = 1.f / l_w;
+  uint16_t* const op =
+      static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(b) * a.T + t_w + n) * a.o_rs + h * a.o_hs + 64 * hf;
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+    for (int r8 = 0; r8 < 2; ++r8) {
+      uint32_t o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = pack_bf16x2(oacc[cb][8 * r8 + 2 * e] * inv, oacc[cb][8 * r8 + 2 * e + 1] * inv);
+      *reinterpret_cast<uint4*>(op + 16 * cb + 8 * r8) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+}  // namespace
+
+int launch_prompt(const PromptArgs& a, hipStream_t s) {
+  if (a.B == 0 || a.T == 0 || a.H == 0) return 0;
+  const int64_t blocks = static_cast<int64_t>((a.T + kPrQ - 1) / kPrQ) * a.B * a.H;
+  if (blocks > (int64_t(1) << 31) - 1) return -1;
+  hipLaunchKernelGGL(mla_prompt_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kPrWaves * 64), 0, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+}  // namespace swamla

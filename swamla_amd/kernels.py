@@ -562,13 +562,23 @@ def head_product_ok(K: int, N: int) -> bool:
     return 64 <= K <= 512 and K % 64 == 0 and N > 0 and N % 4 == 0
 
 
-def head_product(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+def head_product(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
+                 scale: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[m, h, n] = x[m, h, :] . w[h, n, :] in bf16 with fp32 accumulation
     and one rounding (mla_head_product), for prompt-sized row counts: the
     absorbed products q_nope . W_uk and o_lat . W_uv^T that re-associate the
     einsums of models/mla.py:427 and :433.  x [M, H, K], w [H, N, K] and out
     [M, H, N] may be strided views with a unit last stride (x read in place,
-    e.g. the q_nope columns of the wq output)."""
+    e.g. the q_nope columns of the wq output).
+
+    Rows that every head shares (mla_head_product_rows): x [B, 1, M, K] cache
+    rows, out [B, H, M, N], the einsums as written (a head's keys and values
+    of cached latents); x may then hold e4m3 codes (uint8) with ``scale``
+    [B, M] fp32, one per row."""
+    if x.dim() == 4:
+        return _head_product_rows(x, w, out, scale)
+    if scale is not None:
+        raise ValueError("row scales need x [B, 1, M, K]")
     dev = _need_gpu(x, w, out)
     if x.dim() != 3 or w.dim() != 3 or x.shape[1] != w.shape[0] or x.shape[2] != w.shape[2]:
         raise ValueError(f"x {tuple(x.shape)} and w {tuple(w.shape)} must be [M, H, K] / [H, N, K]")
@@ -588,6 +598,150 @@ def head_product(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] =
             x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(), w.stride(1), w.stride(0),
             out.data_ptr(), out.stride(0), out.stride(1), M, N, K, Hx,
             _abi.DTYPE_BF16, _abi.stream_handle(dev),
+        )
+    )
+    return out
+
+
+def _head_product_rows(x, w, out, scale):
+    dev = _need_gpu(x, w, out, scale)
+    fp8 = x.dtype == torch.uint8
+    if x.shape[1] != 1 or w.dim() != 3 or x.shape[3] != w.shape[2]:
+        raise ValueError(f"x {tuple(x.shape)} and w {tuple(w.shape)} must be [B, 1, M, K] / [H, N, K]")
+    if not (fp8 or x.dtype == torch.bfloat16) or w.dtype != torch.bfloat16:
+        raise TypeError("head_product: bf16 weights, bf16 rows or e4m3 codes")
+    B, _, M, K = x.shape
+    Hx, N = w.shape[:2]
+    if fp8 != (scale is not None) or (fp8 and (scale.dtype != torch.float32 or tuple(scale.shape) != (B, M)
+                                               or (M > 1 and scale.stride(1) != 1))):
+        raise ValueError("e4m3 rows need a float32 scale [B, M] with unit last stride (and only they)")
+    if out is None:
+        out = torch.empty(B, Hx, M, N, dtype=torch.bfloat16, device=dev)
+    if tuple(out.shape) != (B, Hx, M, N) or out.dtype != torch.bfloat16:
+        raise ValueError(f"out must be [{B}, {Hx}, {M}, {N}] bf16")
+    for t, name in ((x, "x"), (w, "w"), (out, "out")):
+        if t.stride(-1) != 1:
+            raise ValueError(f"{name} needs a unit last stride")
+    _abi.check(
+        _abi.lib().mla_head_product_rows(
+            x.data_ptr(), x.stride(2), x.stride(0), _abi.ptr(scale), scale.stride(0) if fp8 else 0,
+            w.data_ptr(), w.stride(1), w.stride(0), out.data_ptr(), out.stride(2), out.stride(1), out.stride(0),
+            B, M, N, K, Hx, _abi.DTYPE_FP8 if fp8 else _abi.DTYPE_BF16, _abi.stream_handle(dev),
+        )
+    )
+    return out
+
+
+def expanded_ok(rank_pad: int, nope: int, v_dim: int) -> bool:
+    """Whether prompt_attention and the products that feed it cover a layer
+    of this geometry."""
+    return rank_pad <= MAX_RANK and nope == 128 and v_dim == 128 and head_product_ok(nope, v_dim)
+
+
+def use_expanded(n_seq: int, tokens_per_seq: int, start: int, heads: int, rank: int, fp8: bool = False,
+                 num_cus: int = 256) -> bool:
+    """Whether a prompt of ``tokens_per_seq`` tokens per sequence behind
+    ``start`` cached ones is better served by expanded keys and values
+    (prompt_attention) than by attention in the latent space.
+
+    Expanding costs a product over every cached token and makes a (query,
+    key) pair cost 640 flops per head; the latent space costs a product over
+    the new tokens only and 4 R_pad + 128 flops per pair (more in effect
+    above rank 256, where the per-row decode kernel serves it).  Both sides
+    are estimated in microseconds on 256 CUs from measured launches (bf16,
+    16 heads unless said):
+      expanded   keys + values 19 us (512 tokens), 61 (16,384), 60 (8,008 at
+                 rank 444), 119 (8,192 at rank 1000); attention 17 us
+                 (1 x 512), 63 (8 x 1001), 410 (4 x 4096): about 3 us per
+                 64-token tile of a workgroup, two workgroups per CU
+      latent     products 10 us + 4 us per 1,000 tokens; 20 us per million
+                 pairs (bf16 cache of 128 or 256 padded channels, prefill
+                 kernel), 38 (the others up to 256), 44 (rank / 256)^1.2 plus
+                 0.03 us per row on the decode kernel, twice that above 512
+    Whole forwards at the crossing (expanded / latent, us): 1 x 256 from 0
+    70 / 64, 1 x 512 77 / 79, 32 x 64 at 1024 254 / 141, 8 x 512 at 4096
+    437 / 431, 1 x 256 at 4096 169 / 111, 2 x 512 at 8192 301 / 447.  A gain
+    of less than 5 us does not move a call off the latent path."""
+    B, T, L = n_seq, tokens_per_seq, start + tokens_per_seq
+    rp = padded_rank(rank)
+    width = max(rp, 256) / 256.0
+    tiles = [-(-(start + min(T, t + 128)) // 64) for t in range(0, T, 128)]
+    expand = 14 + 3.0e-3 * B * L * heads / 16 * width
+    attn = max(5 + 1.3 * tiles[-1], B * heads * sum(3 + 3.05 * t for t in tiles) / (2 * num_cus))
+    pairs = B * (T * start + T * (T + 1) / 2) * 1e-6
+    rows = B * T
+    if use_prefill(B, T, num_cus, rank):
+        launches = -(-heads // H)
+        m32 = not fp8 and rp % 128 == 0
+        latent = 10 + pairs * launches * (20 if m32 else 38) * (4 * rp + 128) / 1152
+    else:
+        launches = 1 if heads == 2 * H and rp <= 256 else -(-heads // H)
+        latent = launches * (0.03 * rows + 44 * pairs * (rp / 256) ** 1.2) * (2 if rp > MFMA_MAX_RANK else 1)
+        if launches == 1 and heads > H:
+            latent *= 1.3
+    if heads % H != 0:
+        latent += 4  # query heads zero-padded to whole launches
+    latent += 10 + 4.0e-3 * rows * heads / 16
+    return expand + attn + 5 < latent
+
+
+def prompt_value_order(device=None) -> torch.Tensor:
+    """The channel that each of the 128 positions of prompt_attention's value
+    rows holds (position 32 c + 8 a + 4 f + e: channel 64 f + 16 c + 4 a + e,
+    so that a lane of the kernel ends up with consecutive channels)."""
+    p = torch.arange(128, device=device)
+    return 64 * ((p >> 2) & 1) + 16 * (p >> 5) + 4 * ((p >> 3) & 3) + (p & 3)
+
+
+def prompt_attention(
+    q: torch.Tensor,
+    cos_tab: torch.Tensor,
+    sin_tab: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    cache: LatentCache,
+    sm_scale: float,
+    *,
+    start: int,
+    tokens_per_seq: int,
+    rope_abs: bool = False,
+    out: Optional[torch.Tensor] = None,
+) -> torch.Tensor:
+    """Causal attention of T = ``tokens_per_seq`` new tokens per sequence, all
+    from position ``start``, over expanded keys and values (mla_prompt_attn):
+    token t attends to [0, start + t].  q [B * T, H, 192] (nope | rope,
+    unrotated; may be a strided view), k and v [B, H, start + T, 128]
+    contiguous (head_product of the cache rows with W_uk and with W_uv's rows
+    in prompt_value_order), k_pe from ``cache``; returns [B * T, H, 128].
+    Reference: models/mla.py:427-487."""
+    cache.validate()
+    dev = _need_gpu(q, cos_tab, sin_tab, k, v, cache.kpe, out)
+    T, L = int(tokens_per_seq), int(start) + int(tokens_per_seq)
+    n, nh = q.shape[0], q.shape[1]
+    if T < 1 or n % T != 0 or start < 0:
+        raise ValueError(f"{n} rows of {T} tokens per sequence from position {start}")
+    B = n // T
+    if q.dim() != 3 or q.shape[2] != 192 or q.stride(2) != 1:
+        raise ValueError("q must be [B * T, H, 192] with a unit last stride")
+    for t, name in ((k, "k"), (v, "v")):
+        if tuple(t.shape) != (B, nh, L, 128) or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous [{B}, {nh}, {L}, 128] tensor")
+    if any(t.dtype != torch.bfloat16 for t in (q, k, v, cos_tab, sin_tab, cache.kpe)):
+        raise TypeError("prompt_attention: bf16 tensors only")
+    if cos_tab.dim() != 2 or cos_tab.shape[1] != P // 2 or cos_tab.shape != sin_tab.shape:
+        raise ValueError("RoPE tables must be [S, P/2]")
+    if not (cos_tab.is_contiguous() and sin_tab.is_contiguous()):
+        raise ValueError("RoPE tables must be contiguous")
+    if out is None:
+        out = torch.empty(n, nh, 128, dtype=q.dtype, device=dev)
+    if tuple(out.shape) != (n, nh, 128) or out.dtype != q.dtype or out.stride(2) != 1:
+        raise ValueError(f"out must be [{n}, {nh}, 128] bf16 with a unit last stride")
+    _abi.check(
+        _abi.lib().mla_prompt_attn(
+            q.data_ptr(), q.stride(0), q.stride(1), cos_tab.data_ptr(), sin_tab.data_ptr(), cos_tab.shape[0],
+            k.data_ptr(), v.data_ptr(), cache.kpe.data_ptr(), cache.kpe.shape[0], cache.kpe.shape[1],
+            B, T, int(start), int(bool(rope_abs)), nh, 128, P, 128, float(sm_scale),
+            out.data_ptr(), out.stride(0), out.stride(1), _abi.DTYPE_BF16, _abi.stream_handle(dev),
         )
     )
     return out

@@ -374,6 +374,20 @@ class MLA(nn.Module):
             self._padded_w["w_uk_t"] = hit
         return hit[1]
 
+    def _w_expand(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """W_uk [H, nope, R_pad] and W_uv [H, Dv, R_pad] with W_uv's rows in
+        prompt_attention's order of value channels: what expands a cached
+        latent into its heads' keys and values (mla.py:427-437)."""
+        H, Dn, Dv, R = self.n_heads, self.qk_nope_head_dim, self.v_head_dim, self.kv_lora_rank
+        src = self.wkv_b.weight
+        view = lambda: src.detach().view(H, Dn + Dv, R)
+        w_uk = view()[:, :Dn] if self.rank_pad == R else self._derived(
+            "w_uk.expand", src, lambda: kernels.pad_rank(view()[:, :Dn], R))
+        w_uv = self._derived(
+            "w_uv.expand", src,
+            lambda: kernels.pad_rank(view()[:, Dn:].index_select(1, kernels.prompt_value_order(src.device)), R))
+        return w_uk, w_uv
+
     # ------------------------------------------------------------- weights
     def absorbed_weights(self) -> tuple[torch.Tensor, torch.Tensor]:
         """W_uk [H, nope, R_pad] and W_uv^T [H, R_pad, v] from wkv_b
@@ -581,10 +595,13 @@ class MLA(nn.Module):
                 f"qk_rope_head_dim={self.qk_rope_head_dim}"
             )
 
-    def _split_plan(self, n_rows: int, max_len: int, device, blocks_per_cu: int = 1) -> tuple[int, int]:
+    def _cus(self, device) -> int:
         if self._num_cus is None:
             self._num_cus = torch.cuda.get_device_properties(device).multi_processor_count
-        return kernels.plan_splits(n_rows, max_len, num_cus=self._num_cus, blocks_per_cu=blocks_per_cu)
+        return self._num_cus
+
+    def _split_plan(self, n_rows: int, max_len: int, device, blocks_per_cu: int = 1) -> tuple[int, int]:
+        return kernels.plan_splits(n_rows, max_len, num_cus=self._cus(device), blocks_per_cu=blocks_per_cu)
 
     def _decode_plan(self, n_rows: int, max_len: int, device, per_row_positions: bool,
                      dtype: Optional[torch.dtype] = None) -> tuple[int, int, int]:
@@ -759,6 +776,35 @@ class MLA(nn.Module):
             raise ValueError(f"start_pos {start_pos} + seqlen {T} exceeds max_seq_len {cache.ckv.shape[1]}")
         return torch.full((B,), start_pos, dtype=torch.int32, device=device)
 
+    # Keys and values of a prompt are expanded for as many sequences at a time
+    # as fit this many bytes (at least one).
+    EXPAND_BYTES = 512 << 20
+
+    def _expanded_attention(self, q: torch.Tensor, cache: LatentCache, cos: torch.Tensor, sin: torch.Tensor,
+                            B: int, T: int, start: int, rope_abs: bool) -> torch.Tensor:
+        """Attention output [B * T, H, Dv] of a prompt (q [B * T, H, 192] from
+        position ``start``, its own tokens already in the cache): cached
+        latents expanded into each head's keys and values once, then causal
+        attention over them (mla.py:427-487)."""
+        H, L = self.n_heads, start + T
+        w_uk, w_uv = self._w_expand()
+        o = torch.empty(B * T, H, self.v_head_dim, dtype=q.dtype, device=q.device)
+        per_seq = 2 * H * L * 128 * q.element_size()
+        step = min(B, max(1, self.EXPAND_BYTES // per_seq))
+        kv = torch.empty(2, step, H, L, 128, dtype=q.dtype, device=q.device)
+        for b0 in range(0, B, step):
+            b1 = min(B, b0 + step)
+            part = LatentCache(cache.ckv[b0:b1], cache.kpe[b0:b1],
+                               None if cache.scale is None else cache.scale[b0:b1], cache.rank)
+            k, v = kv[0, : b1 - b0], kv[1, : b1 - b0]
+            rows = part.ckv[:, None, :L]
+            scale = None if part.scale is None else part.scale[:, :L]
+            kernels.head_product(rows, w_uk, out=k, scale=scale)
+            kernels.head_product(rows, w_uv, out=v, scale=scale)
+            kernels.prompt_attention(q[b0 * T: b1 * T], cos, sin, k, v, part, self.softmax_scale, start=start,
+                                     tokens_per_seq=T, rope_abs=rope_abs, out=o[b0 * T: b1 * T])
+        return o
+
     def _forward_kernels(self, x: torch.Tensor, start_pos) -> torch.Tensor:
         B, T, _ = x.size()
         dev = x.device
@@ -802,6 +848,16 @@ class MLA(nn.Module):
         if not fold_append:
             kernels.append(kv, cache, ln_w, ln_b, self.kv_norm.eps, cos, sin,
                            start_pos=sp, tokens_per_seq=T, rope_abs=rope_abs, err_flag=err)
+
+        # A prompt whose start is known on the host, where its queries attend
+        # to about as many tokens as there are queries: keys and values
+        # expanded per head, as the reference does.
+        if (not fused and T > 1 and x.dtype == torch.bfloat16 and kernels.expanded_ok(self.rank_pad, Dn, Dv)
+                and not (self.inference_mode and isinstance(start_pos, torch.Tensor))):
+            start = int(start_pos) if self.inference_mode else 0
+            if kernels.use_expanded(B, T, start, H, R, self.fp8_cache, self._cus(dev)):
+                o = self._expanded_attention(q, cache, cos, sin, B, T, start, rope_abs)
+                return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
 
         n_splits, min_chunk, balance = self._decode_plan(
             n, max_len, dev, isinstance(start_pos, torch.Tensor) and self.inference_mode, dtype=x.dtype)
