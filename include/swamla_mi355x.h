@@ -377,6 +377,18 @@ int mla_merge_project(const float* o_part, const float* lse_part,
                       int64_t w_rs, int64_t w_hs, int32_t Dv, void* y,
                       int64_t y_rs, int64_t y_hs, int32_t dtype, void* stream);
 
+/* mla_merge_project_wide — the same for kv_lora_rank 513 .. 1024. */
+int mla_merge_project_wide(const float* o_part, const float* lse_part,
+                           const void* o_lat, int64_t o_rs, int64_t o_hs,
+                           const int32_t* kv_len, const int32_t* row_seq,
+                           const int32_t* start_pos, int32_t rows_per_seq,
+                           int64_t cache_batch, int64_t cache_seq,
+                           int32_t n_rows, int32_t H, int32_t R,
+                           int32_t n_splits, int32_t min_chunk,
+                           const int32_t* plan, const void* w, int64_t w_rs,
+                           int64_t w_hs, int32_t Dv, void* y, int64_t y_rs,
+                           int64_t y_hs, int32_t dtype, void* stream);
+
 /*
  * mla_head_product — the per-head products of the prompt pass (prefill-side
  * absorption): y[m][h][n] = sum_k x[m][h][k] * w[h][n][k] for m < M, h < H,

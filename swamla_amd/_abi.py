@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "mla_pack_weight",
     "mla_linear_packed",
     "mla_merge_project",
+    "mla_merge_project_wide",
     "mla_head_product",
     "mla_head_product_rows",
     "mla_prompt_attn",
@@ -123,11 +124,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.mla_linear.argtypes = [
         _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P,
     ]
-    lib.mla_merge_project.restype = ctypes.c_int
-    lib.mla_merge_project.argtypes = [
-        _P, _P, _P, _I64, _I64, _P, _P, _P, _I32, _I64, _I64, _I32, _I32, _I32, _I32, _I32,
-        _P, _P, _I64, _I64, _I32, _P, _I64, _I64, _I32, _P,
-    ]
+    for name in ("mla_merge_project", "mla_merge_project_wide"):
+        getattr(lib, name).restype = ctypes.c_int
+        getattr(lib, name).argtypes = [
+            _P, _P, _P, _I64, _I64, _P, _P, _P, _I32, _I64, _I64, _I32, _I32, _I32, _I32, _I32,
+            _P, _P, _I64, _I64, _I32, _P, _I64, _I64, _I32, _P,
+        ]
     lib.mla_head_product.restype = ctypes.c_int
     lib.mla_head_product.argtypes = [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _P]
     lib.mla_head_product_rows.restype = ctypes.c_int

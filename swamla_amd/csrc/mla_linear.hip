@@ -122,20 +122,22 @@ __global__ __launch_bounds__(NW * 64) void mla_linear_kernel(LinearArgs a) {
 
 
 // ---------------------------------------------------------------------------
-// Split merge + W_uv read-out.  Block = (ROWS query rows, head h), 4 waves;
-// ROWS (2, 4 or 8) keeps the grid near one block per CU.
-// The block first issues its W_uv[h] loads (wave w: output tiles w and w+4,
+// Split merge + W_uv read-out.  Block = (ROWS query rows, head h), 4 waves (8
+// above R_pad = 512: one output tile per wave, whose W_uv rows of up to 1024
+// values are then 128 registers); ROWS (2, 4 or 8) keeps the grid near one
+// block per CU.
+// The block first issues its W_uv[h] loads (wave w: output tiles w, w + NW,
 // all R_pad = 64 NB K; W_uv rows hold R_pad values), then merges its rows'
 // split partials into bf16 rows in LDS (thread t < 32*ROWS: row t/32,
 // channels 8(t%32) + 256k ..+8; one split: the decode kernel's o_lat row),
 // then multiplies: y[r, h, d] = sum_c W_uv[h][d][c] x[r][c].
 // ---------------------------------------------------------------------------
-template <int DV, int ROWS, int NB, int G>
-__global__ __launch_bounds__(256) void mla_merge_project_kernel(MergeProjectArgs a) {
+template <int DV, int ROWS, int NB, int G, int NW = 4>
+__global__ __launch_bounds__(64 * NW) void mla_merge_project_kernel(MergeProjectArgs a) {
   constexpr int R = 64 * NB;  // R: the padded latent width R_pad
   const int H = a.H;          // heads (16 or 32)
   constexpr int kMpXRow = 2 * R + 16;  // LDS bytes per merged row (padded)
-  constexpr int kTilesPerWave = DV / 16 / 4;
+  constexpr int kTilesPerWave = DV / 16 / NW;
   static_assert(ROWS == 2 || ROWS == 4 || ROWS == 8, "rows per block");
   __shared__ __attribute__((aligned(16))) uint8_t x_lds[ROWS * kMpXRow];
   // group states of the split merge (8 = groups x rows): M, T and A per channel
@@ -160,13 +162,13 @@ __global__ __launch_bounds__(256) void mla_merge_project_kernel(MergeProjectArgs
   auto load_w = [&]() {
 #pragma unroll
     for (int j = 0; j < kTilesPerWave; ++j) {
-      const int d = 16 * (w + 4 * j) + n;
+      const int d = 16 * (w + NW * j) + n;
       const uint16_t* wp = static_cast<const uint16_t*>(a.w) + h * a.w_hs + static_cast<int64_t>(d) * a.w_rs + 8 * g;
 #pragma unroll
       for (int s = 0; s < 2 * NB; ++s) wb[j][s] = *reinterpret_cast<const uint4*>(wp + 32 * s);
     }
   };
-  // Merge.  The block's threads form 8 / ROWS groups of ROWS * 32 (whole
+  // Merge.  The block's threads form groups of ROWS * 32 (whole
   // waves), of which the first G merge: group grp takes splits grp, grp + G,
   // grp + 2G, ... of every row (G > 1 when rows may have more than 8 splits,
   // so their loads go out from several waves at once instead of in rounds of
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(256) void mla_merge_project_kernel(MergeProjectArgs
   if (4 * g < ROWS) {
 #pragma unroll
     for (int j = 0; j < kTilesPerWave; ++j) {
-      const int d = 16 * (w + 4 * j) + n;
+      const int d = 16 * (w + NW * j) + n;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = r0 + 4 * g + i;
@@ -601,21 +603,28 @@ int launch_pack_weight(const PackWeightArgs& a, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+namespace {
+template <int NB, int NW>
+void launch_merge_project_nb(const MergeProjectArgs& a, int rows, hipStream_t s) {
+  const dim3 grid((a.n_rows + rows - 1) / rows, a.H), block(64 * NW);
+  // more than 8 splits per row: every wave of the block takes a share of them
+  const bool many = a.n_splits > 8;
+  if (rows == 2 && many) hipLaunchKernelGGL((mla_merge_project_kernel<128, 2, NB, 4, NW>), grid, block, 0, s, a);
+  else if (rows == 2) hipLaunchKernelGGL((mla_merge_project_kernel<128, 2, NB, 1, NW>), grid, block, 0, s, a);
+  else if (rows == 4 && many) hipLaunchKernelGGL((mla_merge_project_kernel<128, 4, NB, 2, NW>), grid, block, 0, s, a);
+  else if (rows == 4) hipLaunchKernelGGL((mla_merge_project_kernel<128, 4, NB, 1, NW>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((mla_merge_project_kernel<128, 8, NB, 1, NW>), grid, block, 0, s, a);
+}
+}  // namespace
+
 int launch_merge_project(const MergeProjectArgs& a, hipStream_t s) {
   if (a.n_rows == 0) return 0;
   // rows per block: about one (rows, head) block per CU; every block reads
   // its head's whole W_uv slice, so fewer rows mean more re-reads of it
   const int rows = a.n_rows * a.H <= 2 * 256 ? 2 : (a.n_rows * a.H <= 4 * 256 ? 4 : 8);
-  const dim3 grid((a.n_rows + rows - 1) / rows, a.H), block(256);
-  const int rc = with_nb(a.R, [&](auto nb) {
+  const int rc = with_nb_wide(a.R, [&](auto nb) {
     constexpr int NB = decltype(nb)::value;
-    // more than 8 splits per row: every wave of the block takes a share of them
-    const bool many = a.n_splits > 8;
-    if (rows == 2 && many) hipLaunchKernelGGL((mla_merge_project_kernel<128, 2, NB, 4>), grid, block, 0, s, a);
-    else if (rows == 2) hipLaunchKernelGGL((mla_merge_project_kernel<128, 2, NB, 1>), grid, block, 0, s, a);
-    else if (rows == 4 && many) hipLaunchKernelGGL((mla_merge_project_kernel<128, 4, NB, 2>), grid, block, 0, s, a);
-    else if (rows == 4) hipLaunchKernelGGL((mla_merge_project_kernel<128, 4, NB, 1>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((mla_merge_project_kernel<128, 8, NB, 1>), grid, block, 0, s, a);
+    launch_merge_project_nb<NB, NB <= kMaxNB ? 4 : 8>(a, rows, s);
     return 0;
   });
   if (rc != 0) return rc;

@@ -857,6 +857,21 @@ def merge_project(
     decode call used (``balanced``: the decode call had ``balance`` > 0 and
     left its chunk in ``workspace.plan``).  Reference: models/mla.py:433,
     :490-491."""
+    return _merge_project(_abi.lib().mla_merge_project, o_lat, w_uv, out, cache, n_splits, min_chunk, workspace,
+                          row_seq, kv_len, start_pos, rows_per_seq, balanced)
+
+
+def merge_project_wide(o_lat: torch.Tensor, w_uv: torch.Tensor, out: torch.Tensor, cache: LatentCache, *,
+                       n_splits: int, min_chunk: int, workspace: Optional[DecodeWorkspace] = None,
+                       start_pos: Optional[torch.Tensor] = None, rows_per_seq: int = 1,
+                       balanced: bool = False) -> torch.Tensor:
+    """merge_project for kv_lora_rank above MFMA_MAX_RANK (mla_merge_project_wide)."""
+    return _merge_project(_abi.lib().mla_merge_project_wide, o_lat, w_uv, out, cache, n_splits, min_chunk, workspace,
+                          None, None, start_pos, rows_per_seq, balanced)
+
+
+def _merge_project(entry, o_lat, w_uv, out, cache, n_splits, min_chunk, workspace, row_seq, kv_len, start_pos,
+                   rows_per_seq, balanced):
     dev = _need_gpu(o_lat, w_uv, out, row_seq, kv_len, start_pos)
     rows = o_lat.shape[0]
     Dv = w_uv.shape[1]
@@ -877,7 +892,7 @@ def merge_project(
     if (n_splits > 1 or balanced) and (workspace is None or not workspace.fits(rows, n_splits, rk, nh)):
         raise ValueError("merge_project needs the decode call's workspace")
     _abi.check(
-        _abi.lib().mla_merge_project(
+        entry(
             _abi.ptr(workspace.o_part if n_splits > 1 else None),
             _abi.ptr(workspace.lse_part if n_splits > 1 else None),
             o_lat.data_ptr(), o_lat.stride(0), o_lat.stride(1),

@@ -18,8 +18,15 @@ What runs where (per forward, bf16 model):
     mla_linear_packed  wo
   prompt-sized calls:
     ATen GEMMs         wq / wkv_a / wo
+    mla_append, then, where the queries attend to about as many tokens as
+    there are queries (kernels.use_expanded): mla_head_product_rows twice
+    (cached latents into each head's keys and values) and mla_prompt_attn;
+    else in the latent space:
     mla_head_product   q_abs = q_nope . W_uk and o = o_lat . W_uv^T
     mla_append, then mla_prefill_attn (or mla_decode_attn + mla_merge)
+  above rank 512 a decode-sized call runs one product for q and the wkv_a
+  rows, mla_append, mla_head_product (q_abs), mla_decode_attn,
+  mla_merge_project_wide and wo.
   fp32 models use the ATen products and batched absorption around mla_append
   and the fp32 decode kernel.  The attention launches take 16 heads each,
   and a bf16 decode launch over a bf16 cache of R_pad <= 256 also 32 (two head
@@ -586,6 +593,66 @@ class MLA(nn.Module):
             and self.v_head_dim == 128
         )
 
+    def _wide_step_ok(self, x: torch.Tensor, n: int) -> bool:
+        """The decode step above rank 512: bf16 modules with up to 16 heads of
+        the built dimensions, at most 128 query rows."""
+        q_bias = ([self.wq.bias] if self.q_lora_rank == 0 else [self.wq_a.bias, self.wq_b.bias]) + [self.wkv_a.bias]
+        return (
+            self.rank_pad > kernels.MFMA_MAX_RANK
+            and self.n_heads <= kernels.H
+            and x.dtype == torch.bfloat16
+            and self.wkv_a.weight.dtype == torch.bfloat16
+            and 0 < n <= kernels.LINEAR_MAX_ROWS
+            and self.qk_nope_head_dim == 128
+            and self.v_head_dim == 128
+            and len({b is None for b in q_bias}) == 1
+        )
+
+    def _wide_weights(self):
+        """(weight, bias or None, packed copy or None) of [wq | wkv_a (R_pad +
+        P rows)] over the model width, or of [wq_a | wkv_a] and wq_b; the
+        query rows padded with zeros to the launch's 16 heads."""
+        first = self.wq if self.q_lora_rank == 0 else self.wq_a
+        ws = [first.weight, self.wkv_a.weight, first.bias, self.wkv_a.bias]
+        if self.q_lora_rank > 0:
+            ws += [self.wq_b.weight, self.wq_b.bias]
+        key = tuple(None if t is None else (t.data_ptr(), t._version, t.dtype, t.device) for t in ws)
+        if self._decode_w is None or self._decode_w[0] != key:
+            pk = lambda w: kernels.pack_weight(w) if kernels.packed_ok(1, w.shape[0], w.shape[1]) else None
+            extra = (kernels.H - self.n_heads) * self.qk_head_dim
+            heads = lambda t: torch.cat([t.detach(), t.new_zeros((extra,) + tuple(t.shape[1:]))])
+            wkv_a, bkv_a = self._wkv_a_padded()
+            q1 = heads if self.q_lora_rank == 0 else (lambda t: t.detach())
+            w1 = torch.cat([q1(first.weight), wkv_a]).contiguous()
+            b1 = None if first.bias is None else torch.cat([q1(first.bias), bkv_a]).contiguous()
+            sets = [(w1, b1, pk(w1))]
+            if self.q_lora_rank > 0:
+                w2, b2 = heads(self.wq_b.weight), None if self.wq_b.bias is None else heads(self.wq_b.bias)
+                sets.append((w2, b2, pk(w2)))
+            self._decode_w = (key, sets)
+        return self._decode_w[1]
+
+    def _wide_projections(self, x: torch.Tensor):
+        """q [n, 16, 192] (heads past n_heads zero) and kv [n, R_pad + P] of the
+        decode step above rank 512."""
+        n = x.shape[0] * x.shape[1]
+        sets = self._wide_weights()
+        y = self._product(x.reshape(n, self.dim), *sets[0])
+        nq = sets[0][0].shape[0] - (self.rank_pad + self.qk_rope_head_dim)
+        q = y[:, :nq]
+        if self.q_lora_rank > 0:
+            q = torch.nn.functional.layer_norm(q, (nq,), self.q_norm.weight, self.q_norm.bias, self.q_norm.eps)
+            q = self._product(q, *sets[1])
+        return q.view(n, kernels.H, self.qk_head_dim), y[:, nq:]
+
+    def _w_uk_t_wide(self) -> torch.Tensor:
+        """_w_uk_t() over the launch's 16 heads (zero for the padding heads)."""
+        w, H = self._w_uk_t(), self.n_heads
+        if H == kernels.H:
+            return w
+        return self._derived("w_uk_t.wide", self.wkv_b.weight,
+                             lambda: torch.cat([w, w.new_zeros((kernels.H - H,) + tuple(w.shape[1:]))], 0))
+
     def _check_geometry(self) -> None:
         if (self.n_heads < 1 or self.qk_rope_head_dim != kernels.P
                 or not 1 <= self.kv_lora_rank <= kernels.MAX_RANK):
@@ -683,6 +750,19 @@ class MLA(nn.Module):
             return None
         return sp
 
+    def _fused_output(self, o: torch.Tensor, start_pos, sp: torch.Tensor, B: int, T: int) -> torch.Tensor:
+        """wo over the decode step's o [n, heads * Dv] (mla.py:490-495)."""
+        n = B * T
+        wo_b = None if self.wo.bias is None else self.wo.bias.detach()
+        wo_p = self._packed_wo()
+        if wo_p is not None and kernels.packed_ok(n, wo_p.N, wo_p.K):
+            adv = self._advance_target(start_pos, sp, T)
+            out = kernels.linear_packed(o, wo_p, bias=wo_b, advance=adv).view(B, T, self.dim)
+            self._advance_folded = adv is not None
+        else:
+            out = kernels.linear(o, self._wo_fused(), bias=wo_b).view(B, T, self.dim)
+        return self.resid_dropout(out)
+
     def _is_causal_prompt_mask(self, mask: torch.Tensor, T: int, start_pos) -> bool:
         """True for the mask SWAMLAModel passes with a prompt
         (swa_mla_model.py:207-211, :384-387: triu(full(-inf), 1)[:T, :T],
@@ -734,14 +814,18 @@ class MLA(nn.Module):
         that forward feeds the append kernel (mla.py:281-288, :307-308), with
         zero latent padding up to R_pad.
         Decode-sized bf16 inputs take kv from the fused input product (and
-        return no q: forward uses the absorbed query directly); other inputs
-        use the ATen projections (q is skipped when not needed)."""
+        return no q: forward uses the absorbed query directly), above rank 512
+        q and kv from one product; other inputs use the ATen projections (q is
+        skipped when not needed)."""
         B, T, _ = x.size()
         n, H = B * T, self.n_heads
         with torch.no_grad():
             if self._fused_step_ok(x, n):
                 _, _, kv = self._fused_projections(x)
                 return None, kv
+            if self._wide_step_ok(x, n):
+                q, kv = self._wide_projections(x)
+                return q[:, :H], kv
             if self.rank_pad == self.kv_lora_rank:
                 kv = self.wkv_a(x).view(n, -1)
             else:
@@ -834,8 +918,12 @@ class MLA(nn.Module):
             max_len = T
 
         fused = self._fused_step_ok(x, n)
+        wide = self._wide_step_ok(x, n)
         if fused:
             q_abs, q_pe, kv = self._fused_projections(x)
+        elif wide:
+            q16, kv = self._wide_projections(x)
+            q = q16[:, :H]
         else:
             q, kv = self.input_projections(x)
 
@@ -888,15 +976,24 @@ class MLA(nn.Module):
             o = torch.empty(n, Hp * Dv, dtype=x.dtype, device=dev)
             kernels.merge_project(o_lat, w_uv, o.view(n, Hp, Dv), cache, n_splits=n_splits, min_chunk=min_chunk,
                                   workspace=ws, start_pos=sp, rows_per_seq=T, balanced=balance > 0)
-            wo_b = None if self.wo.bias is None else self.wo.bias.detach()
-            wo_p = self._packed_wo()
-            if wo_p is not None and kernels.packed_ok(n, wo_p.N, wo_p.K):
-                adv = self._advance_target(start_pos, sp, T)
-                out = kernels.linear_packed(o, wo_p, bias=wo_b, advance=adv).view(B, T, self.dim)
-                self._advance_folded = adv is not None
-            else:
-                out = kernels.linear(o, self._wo_fused(), bias=wo_b).view(B, T, self.dim)
-            return self.resid_dropout(out)  # mla.py:490-495
+            return self._fused_output(o, start_pos, sp, B, T)
+
+        if wide and not prefill:
+            # above rank 512: the queries absorbed per head, attention with the
+            # split merge and W_uv read-out in one launch, wo
+            Hp, rp = kernels.H, self.rank_pad
+            q_abs = x.new_empty(n, Hp, rp)
+            kernels.head_product(q16[:, :, :Dn], self._w_uk_t_wide(), out=q_abs)
+            o_lat = x.new_empty(n, Hp, rp)
+            ws = self._workspace_for(n, n_splits, dev)
+            kernels.decode_attention(q_abs, q16[:, :, Dn:], cos, sin, cache, self.softmax_scale, start_pos=sp,
+                                     rows_per_seq=T, rope_abs=rope_abs, n_splits=n_splits, min_chunk=min_chunk, out=o_lat,
+                                     workspace=ws, merge=False, balance=balance)
+            o = x.new_empty(n, Hp * Dv)
+            kernels.merge_project_wide(o_lat, self._w_uv_fused(), o.view(n, Hp, Dv), cache, n_splits=n_splits,
+                                       min_chunk=min_chunk, workspace=ws, start_pos=sp, rows_per_seq=T,
+                                       balanced=balance > 0)
+            return self._fused_output(o, start_pos, sp, B, T)
 
         # Other calls: the absorbed products, then attention.  The attention
         # kernels take 16 heads per launch (the decode kernel also 32), so H
