@@ -457,6 +457,18 @@ int mla_prompt_attn(const void* q, int64_t q_rs, int64_t q_hs,
                     int32_t Dv, float sm_scale, void* out, int64_t o_rs,
                     int64_t o_hs, int32_t dtype, void* stream);
 
+/* mla_prompt_attn_f32 — the same in fp32: kv [B][start + T][H][256]
+ * contiguous (128 key, then 128 value channels in order, the rows
+ * wkv_b(latent) gives); strides multiples of 4. */
+int mla_prompt_attn_f32(const float* q, int64_t q_rs, int64_t q_hs,
+                        const float* cos_tab, const float* sin_tab,
+                        int64_t rope_len, const float* kv,
+                        const float* kpe_cache, int64_t cache_batch,
+                        int64_t cache_seq, int32_t B, int32_t T,
+                        int32_t start, int32_t rope_abs, int32_t H, int32_t Dn,
+                        int32_t P, int32_t Dv, float sm_scale, float* out,
+                        int64_t o_rs, int64_t o_hs, void* stream);
+
 /* Split plan used by both kernels, exported so hosts and tests can size the
  * partial buffers: number of splits of a row of length L (0 for L <= 0). */
 int32_t mla_split_count(int32_t L, int32_t n_splits, int32_t min_chunk);

@@ -47,6 +47,7 @@ EXPORTED_SYMBOLS = (
     "mla_head_product",
     "mla_head_product_rows",
     "mla_prompt_attn",
+    "mla_prompt_attn_f32",
     "mla_host_f32_to_e4m3",
     "mla_host_e4m3_to_f32",
     "mla_host_e4m3x4_to_bf16",
@@ -140,6 +141,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.mla_prompt_attn.argtypes = [
         _P, _I64, _I64, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32,
         _F, _P, _I64, _I64, _I32, _P,
+    ]
+    lib.mla_prompt_attn_f32.restype = ctypes.c_int
+    lib.mla_prompt_attn_f32.argtypes = [
+        _P, _I64, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32,
+        _F, _P, _I64, _I64, _P,
     ]
     lib.mla_host_f32_to_e4m3.restype = None
     lib.mla_host_f32_to_e4m3.argtypes = [_P, _P, _I64]

@@ -649,13 +649,12 @@ int mla_head_product_rows(const void* x, int64_t x_rs, int64_t x_bs, const float
   return ok();
 }
 
-int mla_prompt_attn(const void* q, int64_t q_rs, int64_t q_hs, const void* cos_tab, const void* sin_tab,
-                    int64_t rope_len, const void* k, const void* v, const void* kpe_cache, int64_t cache_batch,
-                    int64_t cache_seq, int32_t B, int32_t T, int32_t start, int32_t rope_abs, int32_t H, int32_t Dn,
-                    int32_t P, int32_t Dv, float sm_scale, void* out, int64_t o_rs, int64_t o_hs, int32_t dtype,
-                    void* stream) {
-  const char* fn = "mla_prompt_attn";
-  if (dtype != SWAMLA_DTYPE_BF16) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: dtype %d not built (bf16 only)", fn, dtype);
+static int prompt_attn(const char* fn, const void* q, int64_t q_rs, int64_t q_hs, const void* cos_tab,
+                       const void* sin_tab, int64_t rope_len, const void* k, const void* v, const void* kpe_cache,
+                       int64_t cache_batch, int64_t cache_seq, int32_t B, int32_t T, int32_t start, int32_t rope_abs,
+                       int32_t H, int32_t Dn, int32_t P, int32_t Dv, float sm_scale, void* out, int64_t o_rs,
+                       int64_t o_hs, int32_t dtype, void* stream) {
+  const bool f32 = dtype == SWAMLA_DTYPE_F32;
   if (Dn != 128 || P != 64 || Dv != 128)
     return fail(SWAMLA_ERR_UNSUPPORTED, "%s: nope %d, rope %d, v %d (built: 128, 64, 128)", fn, Dn, P, Dv);
   if (B < 0 || T < 0 || H < 0 || start < 0)
@@ -672,15 +671,37 @@ int mla_prompt_attn(const void* q, int64_t q_rs, int64_t q_hs, const void* cos_t
   if (q_rs < 0 || q_hs < 192 || o_rs < 0 || o_hs < 128)
     return fail(SWAMLA_ERR_INVALID_ARG, "%s: negative row strides, or head strides below 192 (q) / 128 (out)", fn);
   if (!aligned(q, 16) || !aligned(cos_tab, 8) || !aligned(sin_tab, 8) || !aligned(k, 16) || !aligned(v, 16) ||
-      !aligned(kpe_cache, 16) || !aligned(out, 16) || (q_rs | q_hs | o_rs | o_hs) % 8 != 0)
-    return fail(SWAMLA_ERR_MISALIGNED, "%s: 16-byte aligned bases and strides that are multiples of 8 required", fn);
+      !aligned(kpe_cache, 16) || !aligned(out, 16) || (q_rs | q_hs | o_rs | o_hs) % (f32 ? 4 : 8) != 0)
+    return fail(SWAMLA_ERR_MISALIGNED, "%s: 16-byte aligned bases and strides of whole 16 bytes required", fn);
   const float log2e = 1.4426950408889634f;
   swamla::PromptArgs a{q, q_rs, q_hs, cos_tab, sin_tab, rope_len, k, v, kpe_cache, cache_seq * 64,
                        B, H, T, start, rope_abs, sm_scale * log2e, out, o_rs, o_hs};
-  const int rc = swamla::launch_prompt(a, static_cast<hipStream_t>(stream));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = f32 ? swamla::launch_prompt_f32(a, s) : swamla::launch_prompt(a, s);
   if (rc == -1) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: too many query groups", fn);
   if (rc != 0) return hip_fail(fn);
   return ok();
+}
+
+int mla_prompt_attn(const void* q, int64_t q_rs, int64_t q_hs, const void* cos_tab, const void* sin_tab,
+                    int64_t rope_len, const void* k, const void* v, const void* kpe_cache, int64_t cache_batch,
+                    int64_t cache_seq, int32_t B, int32_t T, int32_t start, int32_t rope_abs, int32_t H, int32_t Dn,
+                    int32_t P, int32_t Dv, float sm_scale, void* out, int64_t o_rs, int64_t o_hs, int32_t dtype,
+                    void* stream) {
+  const char* fn = "mla_prompt_attn";
+  if (dtype != SWAMLA_DTYPE_BF16) return fail(SWAMLA_ERR_UNSUPPORTED, "%s: dtype %d not built (bf16 only)", fn, dtype);
+  return prompt_attn(fn, q, q_rs, q_hs, cos_tab, sin_tab, rope_len, k, v, kpe_cache, cache_batch, cache_seq, B, T,
+                     start, rope_abs, H, Dn, P, Dv, sm_scale, out, o_rs, o_hs, dtype, stream);
+}
+
+int mla_prompt_attn_f32(const float* q, int64_t q_rs, int64_t q_hs, const float* cos_tab, const float* sin_tab,
+                        int64_t rope_len, const float* kv, const float* kpe_cache, int64_t cache_batch,
+                        int64_t cache_seq, int32_t B, int32_t T, int32_t start, int32_t rope_abs, int32_t H,
+                        int32_t Dn, int32_t P, int32_t Dv, float sm_scale, float* out, int64_t o_rs, int64_t o_hs,
+                        void* stream) {
+  return prompt_attn("mla_prompt_attn_f32", q, q_rs, q_hs, cos_tab, sin_tab, rope_len, kv, kv, kpe_cache, cache_batch,
+                     cache_seq, B, T, start, rope_abs, H, Dn, P, Dv, sm_scale, out, o_rs, o_hs, SWAMLA_DTYPE_F32,
+                     stream);
 }
 
 // ---- host-side test hooks: the kernels' bit-level conversions run on the CPU.

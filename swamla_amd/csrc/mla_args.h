@@ -207,6 +207,8 @@ int launch_linear_packed(const PackedLinearArgs& a, hipStream_t s);
 int launch_pack_weight(const PackWeightArgs& a, hipStream_t s);
 int launch_merge_project(const MergeProjectArgs& a, hipStream_t s);
 int launch_prompt(const PromptArgs& a, hipStream_t s);
+// fp32: k holds [B, start + T, H, 256] rows of 128 key, then 128 value channels (in order); v is not read.
+int launch_prompt_f32(const PromptArgs& a, hipStream_t s);
 // -1: no kernel for this K; -2: launch error.
 int launch_head_product(const HeadProductArgs& a, int n_cus, hipStream_t s);
 

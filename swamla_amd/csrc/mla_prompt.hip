@@ -287,7 +287,182 @@ __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same attention for fp32 models (fp32 keys, values, products and sums).
+//
+// Bound: the fp32 matrix rate (32x32x2: 64 cycles for 4,096 flops), and for
+// the shapes it serves the longest chain: one 32-query block of a 512-token
+// prompt is 16 tiles of 160 MFMAs.  A workgroup therefore is eight waves on
+// one block of 32 queries of a (sequence, head), each wave taking every
+// eighth 32-token tile with an online softmax of its own; the eight states are
+// folded through LDS in wave order.
+//   S^T[32 tok x 32 q]: k slot (step e of 8-channel group g, lane half f) is
+//       channel 8 g + 4 f + e, so a lane's operands of four steps are 16
+//       consecutive bytes of its row (K from global memory, each row used by
+//       one wave only; Q from LDS, shared by the eight waves).
+//   O^T[32 x 32 q]: k slot (register r = 4 a + e, half f) is token 8 a + 4 f + e,
+//       the score registers as they are; block i's row m is channel 4 m + i,
+//       so one 16-byte load of a V row serves the four blocks.
+// Measured, 1 x 512 tokens, 16 heads: 32 us against 484 for the per-row VALU
+// kernel (the longest block's 16 tiles are two per wave: 9 us of MFMAs).
+constexpr int kPfWaves = 8;
+constexpr int kPfQPitch = 196;  // floats per Q row: 49 16-byte chunks, so 16 rows of a read hit distinct banks
+
+__global__ __launch_bounds__(kPfWaves * 64, 2) void mla_prompt_f32_kernel(PromptArgs a) {
+  __shared__ __attribute__((aligned(16))) float q_lds[32 * kPfQPitch];
+  __shared__ __attribute__((aligned(16))) float o_lds[kPfWaves][32 * kPrD];
+  __shared__ float m_lds[kPfWaves][32], l_lds[kPfWaves][32];
+
+  const int BH = a.B * a.H;
+  const int n_qb = (a.T + 31) / 32;
+  const int qb_i = n_qb - 1 - static_cast<int>(blockIdx.x) / BH, bh = static_cast<int>(blockIdx.x) % BH;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63, n = lane & 31, hf = lane >> 5;
+  const int t0q = 32 * qb_i;
+  const int L = a.start + min(t0q + 32, a.T);  // the block's causal range
+  const int Lq = a.start + min(t0q + n, a.T - 1) + 1;
+
+  // ---- Q, rotated, into LDS (rows past the last repeat it)
+  for (int i = threadIdx.x; i < 32 * 48; i += kPfWaves * 64) {
+    const int r = i / 48, c = 4 * (i - 48 * r);
+    const int t = min(t0q + r, a.T - 1);
+    float4 v = *reinterpret_cast<const float4*>(static_cast<const float*>(a.q) +
+                                                (static_cast<int64_t>(b) * a.T + t) * a.q_rs + h * a.q_hs + c);
+    if (c >= kPrD) {
+      int rp = a.rope_abs ? a.start + t : t;
+      rp = rp >= a.rope_len ? static_cast<int>(a.rope_len) - 1 : rp;
+      const int64_t o = static_cast<int64_t>(rp) * (kP / 2) + (c - kPrD) / 2;
+      const float2 cs = *reinterpret_cast<const float2*>(static_cast<const float*>(a.cos_tab) + o);
+      const float2 sn = *reinterpret_cast<const float2*>(static_cast<const float*>(a.sin_tab) + o);
+      float4 u;
+      rope_pair<0>(v.x, v.y, cs.x, sn.x, u.x, u.y);
+      rope_pair<0>(v.z, v.w, cs.y, sn.y, u.z, u.w);
+      v = u;
+    }
+    *reinterpret_cast<float4*>(q_lds + r * kPfQPitch + c) = v;
+  }
+  __syncthreads();
+
+  const int n_tiles = (L + 31) / 32;
+  f32x16_t oacc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) oacc[i] = f32x16_t{};
+  float m_run = -INFINITY, l_run = 0.f;
+  const float* const qr = q_lds + n * kPfQPitch + 4 * hf;
+  const int64_t row = static_cast<int64_t>(a.H) * 2 * kPrD;  // floats per token of the expanded rows
+  const float* const kvb = static_cast<const float*>(a.k) + (static_cast<int64_t>(b) * (a.start + a.T) * a.H + h) * 2 * kPrD;
+  const float* const peb = static_cast<const float*>(a.kpe) + static_cast<int64_t>(b) * a.kpe_bs;
+  for (int j = w; j < n_tiles; j += kPfWaves) {
+    const int tok = min(32 * j + n, L - 1);
+    const float* const kp = kvb + tok * row + 4 * hf;
+    const float* const pp = peb + static_cast<int64_t>(tok) * kP + 4 * hf;
+    float4 kr[3][8];
+    auto load = [&](auto B3) __attribute__((always_inline)) {
+      constexpr int c = decltype(B3)::value;
+#pragma unroll
+      for (int g = 0; g < 8; ++g)
+        kr[c][g] = *reinterpret_cast<const float4*>(c < 2 ? kp + 64 * c + 8 * g : pp + 8 * g);
+    };
+    f32x16_t sc = f32x16_t{};
+    load(std::integral_constant<int, 0>{});
+    float4 vr[16];
+    st_for<0, 3>([&](auto C) __attribute__((always_inline)) {
+      constexpr int c = decltype(C)::value;
+      if constexpr (c < 2) {
+        load(std::integral_constant<int, c + 1>{});
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          vr[r] = *reinterpret_cast<const float4*>(
+              kvb + min(32 * j + 8 * (r >> 2) + 4 * hf + (r & 3), L - 1) * row + kPrD + 4 * n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const float4 q4 = *reinterpret_cast<const float4*>(qr + 64 * c + 8 * g);
+        const float4 k4 = kr[c][g];
+        sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, q4.x, sc, 0, 0, 0);
+        sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, q4.y, sc, 0, 0, 0);
+        sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, q4.z, sc, 0, 0, 0);
+        sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, q4.w, sc, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    float mt = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      sc[r] = 32 * j + 8 * (r >> 2) + 4 * hf + (r & 3) < Lq ? sc[r] * a.scale_log2 : -INFINITY;
+      mt = fmaxf(mt, sc[r]);
+    }
+    mt = fmaxf(mt, shfl_xor_f32(mt, 32));
+    const float m_new = fmaxf(m_run, mt);
+    if (__any(m_new > m_run)) {
+      const float alpha = m_new == m_run ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);  // both -inf: 1, not NaN
+      l_run *= alpha;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) oacc[i] *= alpha;
+      m_run = m_new;
+    }
+    const float mref = m_new == -INFINITY ? 0.f : m_new;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      sc[r] = __builtin_amdgcn_exp2f(sc[r] - mref);
+      l_run += sc[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      oacc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].x, sc[r], oacc[0], 0, 0, 0);
+      oacc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].y, sc[r], oacc[1], 0, 0, 0);
+      oacc[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].z, sc[r], oacc[2], 0, 0, 0);
+      oacc[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r].w, sc[r], oacc[3], 0, 0, 0);
+    }
+  }
+
+  // ---- fold the waves that had a tile: weights 2^(m_w - m), sums in wave order
+  const int nw = min(kPfWaves, n_tiles);
+  l_run += shfl_xor_f32(l_run, 32);
+  if (w < nw) {
+    if (hf == 0) {
+      m_lds[w][n] = m_run;
+      l_lds[w][n] = l_run;
+    }
+    // lane (n, hf), register 4 a + e of block i: channel 32 a + 16 hf + 4 e + i
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      *reinterpret_cast<float4*>(&o_lds[w][n * kPrD + ((32 * (r >> 2) + 16 * hf + 4 * (r & 3)) ^ (4 * (n & 7)))]) =
+          make_float4(oacc[0][r], oacc[1][r], oacc[2][r], oacc[3][r]);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 32 * 32; i += kPfWaves * 64) {
+    const int qi = i >> 5, c = 4 * (i & 31);
+    if (t0q + qi >= a.T) continue;
+    float m = -INFINITY;
+    for (int k = 0; k < nw; ++k) m = fmaxf(m, m_lds[k][qi]);
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    float l = 0.f;
+    for (int k = 0; k < nw; ++k) {
+      const float mk = m_lds[k][qi];
+      const float wk = mk == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mk - m);
+      const float4 p = *reinterpret_cast<const float4*>(&o_lds[k][qi * kPrD + (c ^ (4 * (qi & 7)))]);
+      o.x += wk * p.x, o.y += wk * p.y, o.z += wk * p.z, o.w += wk * p.w;
+      l += wk * l_lds[k][qi];
+    }
+    const float inv = 1.f / l;
+    *reinterpret_cast<float4*>(static_cast<float*>(a.out) + (static_cast<int64_t>(b) * a.T + t0q + qi) * a.o_rs +
+                               h * a.o_hs + c) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+  }
+}
+
 }  // namespace
+
+int launch_prompt_f32(const PromptArgs& a, hipStream_t s) {
+  if (a.B == 0 || a.T == 0 || a.H == 0) return 0;
+  const int64_t blocks = static_cast<int64_t>((a.T + 31) / 32) * a.B * a.H;
+  if (blocks > (int64_t(1) << 31) - 1) return -1;
+  hipLaunchKernelGGL(mla_prompt_f32_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kPfWaves * 64), 0, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
 
 int launch_prompt(const PromptArgs& a, hipStream_t s) {
   if (a.B == 0 || a.T == 0 || a.H == 0) return 0;

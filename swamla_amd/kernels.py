@@ -685,6 +685,30 @@ def use_expanded(n_seq: int, tokens_per_seq: int, start: int, heads: int, rank: 
     return expand + attn + 5 < latent
 
 
+def use_expanded_f32(n_seq: int, tokens_per_seq: int, start: int, heads: int, rank: int,
+                     num_cus: int = 256) -> bool:
+    """use_expanded for an fp32 module, whose latent path is the per-row VALU
+    kernel and batched products: only a few tokens behind a long prefix stay
+    there.  Microseconds on 256 CUs, 16 heads, rank 256; whole forwards
+    expanded / latent: 1 x 512 from 0 128 / 608, 1 x 2 46 / 74, 2 x 1024 402 /
+    3070, 1 x 256 at 2000 231 / 2252, 1 x 16 at 4000 299 / 321.  The expansion
+    is a GEMM at about 47 TFLOP/s, a workgroup of the attention takes 5 us per
+    eight tiles; the VALU kernel 3.5 ms per million pairs, and 0.8 us per token
+    of its longest split.  Head counts other than 16 come over from 512 tokens
+    on (1 x 512 at 12 heads 117 / 605); below, they stay on the 16-head
+    launches over padded heads that the tests of those modules count."""
+    B, T, L = n_seq, tokens_per_seq, start + tokens_per_seq
+    if heads != H and B * T < 512:
+        return False
+    rp = padded_rank(rank)
+    pairs = B * (T * start + T * (T + 1) / 2) * 1e-6
+    expand = 10 + 2.0 * B * L * heads * 256 * rp / 47e6
+    attn = max(5 + 5 * -(-L // 256), pairs * heads * 640 / 60)
+    chunk = min(L, max(256, L / -(-num_cus // (B * T))))
+    latent = 25 + -(-heads // H) * rp / 256 * max(3500 * pairs, 0.8 * chunk)
+    return expand + attn < latent
+
+
 def prompt_value_order(device=None) -> torch.Tensor:
     """The channel that each of the 128 positions of prompt_attention's value
     rows holds (position 32 c + 8 a + 4 f + e: channel 64 f + 16 c + 4 a + e,
@@ -714,37 +738,62 @@ def prompt_attention(
     contiguous (head_product of the cache rows with W_uk and with W_uv's rows
     in prompt_value_order), k_pe from ``cache``; returns [B * T, H, 128].
     Reference: models/mla.py:427-487."""
-    cache.validate()
-    dev = _need_gpu(q, cos_tab, sin_tab, k, v, cache.kpe, out)
-    T, L = int(tokens_per_seq), int(start) + int(tokens_per_seq)
-    n, nh = q.shape[0], q.shape[1]
-    if T < 1 or n % T != 0 or start < 0:
-        raise ValueError(f"{n} rows of {T} tokens per sequence from position {start}")
-    B = n // T
-    if q.dim() != 3 or q.shape[2] != 192 or q.stride(2) != 1:
-        raise ValueError("q must be [B * T, H, 192] with a unit last stride")
+    dev, B, nh, L, out = _check_prompt(q, cos_tab, sin_tab, (k, v), cache, start, tokens_per_seq, torch.bfloat16, out)
     for t, name in ((k, "k"), (v, "v")):
         if tuple(t.shape) != (B, nh, L, 128) or not t.is_contiguous():
             raise ValueError(f"{name} must be a contiguous [{B}, {nh}, {L}, 128] tensor")
-    if any(t.dtype != torch.bfloat16 for t in (q, k, v, cos_tab, sin_tab, cache.kpe)):
-        raise TypeError("prompt_attention: bf16 tensors only")
+    _abi.check(
+        _abi.lib().mla_prompt_attn(
+            q.data_ptr(), q.stride(0), q.stride(1), cos_tab.data_ptr(), sin_tab.data_ptr(), cos_tab.shape[0],
+            k.data_ptr(), v.data_ptr(), cache.kpe.data_ptr(), cache.kpe.shape[0], cache.kpe.shape[1],
+            B, int(tokens_per_seq), int(start), int(bool(rope_abs)), nh, 128, P, 128, float(sm_scale),
+            out.data_ptr(), out.stride(0), out.stride(1), _abi.DTYPE_BF16, _abi.stream_handle(dev),
+        )
+    )
+    return out
+
+
+def prompt_attention_f32(q: torch.Tensor, cos_tab: torch.Tensor, sin_tab: torch.Tensor, kv: torch.Tensor,
+                         cache: LatentCache, sm_scale: float, *, start: int, tokens_per_seq: int,
+                         rope_abs: bool = False, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """prompt_attention in fp32 (mla_prompt_attn_f32): kv [B, start + T, H,
+    256] contiguous, 128 key then 128 value channels (wkv_b of the cached
+    latents)."""
+    dev, B, nh, L, out = _check_prompt(q, cos_tab, sin_tab, (kv,), cache, start, tokens_per_seq, torch.float32, out)
+    if tuple(kv.shape) != (B, L, nh, 256) or not kv.is_contiguous():
+        raise ValueError(f"kv must be a contiguous [{B}, {L}, {nh}, 256] tensor")
+    _abi.check(
+        _abi.lib().mla_prompt_attn_f32(
+            q.data_ptr(), q.stride(0), q.stride(1), cos_tab.data_ptr(), sin_tab.data_ptr(), cos_tab.shape[0],
+            kv.data_ptr(), cache.kpe.data_ptr(), cache.kpe.shape[0], cache.kpe.shape[1], B, int(tokens_per_seq),
+            int(start), int(bool(rope_abs)), nh, 128, P, 128, float(sm_scale), out.data_ptr(), out.stride(0),
+            out.stride(1), _abi.stream_handle(dev),
+        )
+    )
+    return out
+
+
+def _check_prompt(q, cos_tab, sin_tab, kvs, cache, start, T, dtype, out):
+    """Shapes of a prompt attention call; (device, sequences, heads, positions, out)."""
+    cache.validate()
+    dev = _need_gpu(q, cos_tab, sin_tab, *kvs, cache.kpe, out)
+    T = int(T)
+    if q.dim() != 3 or q.shape[2] != 192 or q.stride(2) != 1:
+        raise ValueError("q must be [B * T, H, 192] with a unit last stride")
+    n, nh = q.shape[0], q.shape[1]
+    if T < 1 or n % T != 0 or start < 0:
+        raise ValueError(f"{n} rows of {T} tokens per sequence from position {start}")
+    if any(t.dtype != dtype for t in (q, *kvs, cos_tab, sin_tab, cache.kpe)):
+        raise TypeError(f"prompt attention: {dtype} tensors only")
     if cos_tab.dim() != 2 or cos_tab.shape[1] != P // 2 or cos_tab.shape != sin_tab.shape:
         raise ValueError("RoPE tables must be [S, P/2]")
     if not (cos_tab.is_contiguous() and sin_tab.is_contiguous()):
         raise ValueError("RoPE tables must be contiguous")
     if out is None:
-        out = torch.empty(n, nh, 128, dtype=q.dtype, device=dev)
-    if tuple(out.shape) != (n, nh, 128) or out.dtype != q.dtype or out.stride(2) != 1:
-        raise ValueError(f"out must be [{n}, {nh}, 128] bf16 with a unit last stride")
-    _abi.check(
-        _abi.lib().mla_prompt_attn(
-            q.data_ptr(), q.stride(0), q.stride(1), cos_tab.data_ptr(), sin_tab.data_ptr(), cos_tab.shape[0],
-            k.data_ptr(), v.data_ptr(), cache.kpe.data_ptr(), cache.kpe.shape[0], cache.kpe.shape[1],
-            B, T, int(start), int(bool(rope_abs)), nh, 128, P, 128, float(sm_scale),
-            out.data_ptr(), out.stride(0), out.stride(1), _abi.DTYPE_BF16, _abi.stream_handle(dev),
-        )
-    )
-    return out
+        out = torch.empty(n, nh, 128, dtype=dtype, device=dev)
+    if tuple(out.shape) != (n, nh, 128) or out.dtype != dtype or out.stride(2) != 1:
+        raise ValueError(f"out must be [{n}, {nh}, 128] {dtype} with a unit last stride")
+    return dev, n // T, nh, int(start) + T, out
 
 
 PACKED_K = (512, 1024, 1536, 2048)

@@ -889,6 +889,25 @@ class MLA(nn.Module):
                                      tokens_per_seq=T, rope_abs=rope_abs, out=o[b0 * T: b1 * T])
         return o
 
+    def _expanded_attention_f32(self, q: torch.Tensor, cache: LatentCache, cos: torch.Tensor, sin: torch.Tensor,
+                                B: int, T: int, start: int, rope_abs: bool) -> torch.Tensor:
+        """_expanded_attention for an fp32 module: keys and values as wkv_b's
+        product with the cached latents (mla.py:427-437), ATen's GEMM like the
+        module's other fp32 projections."""
+        H, L = self.n_heads, start + T
+        w = self._padded("wkv_b.rank", self.wkv_b.weight,
+                         lambda: kernels.pad_rank(self.wkv_b.weight.detach(), self.kv_lora_rank))
+        o = torch.empty(B * T, H, self.v_head_dim, dtype=q.dtype, device=q.device)
+        per_seq = 2 * H * L * 128 * q.element_size()
+        step = min(B, max(1, self.EXPAND_BYTES // per_seq))
+        for b0 in range(0, B, step):
+            b1 = min(B, b0 + step)
+            part = LatentCache(cache.ckv[b0:b1], cache.kpe[b0:b1], None, cache.rank)
+            kv = torch.nn.functional.linear(part.ckv[:, :L], w).view(b1 - b0, L, H, 256)
+            kernels.prompt_attention_f32(q[b0 * T: b1 * T], cos, sin, kv, part, self.softmax_scale, start=start,
+                                         tokens_per_seq=T, rope_abs=rope_abs, out=o[b0 * T: b1 * T])
+        return o
+
     def _forward_kernels(self, x: torch.Tensor, start_pos) -> torch.Tensor:
         B, T, _ = x.size()
         dev = x.device
@@ -940,11 +959,17 @@ class MLA(nn.Module):
         # A prompt whose start is known on the host, where its queries attend
         # to about as many tokens as there are queries: keys and values
         # expanded per head, as the reference does.
-        if (not fused and T > 1 and x.dtype == torch.bfloat16 and kernels.expanded_ok(self.rank_pad, Dn, Dv)
+        if (not fused and T > 1 and kernels.expanded_ok(self.rank_pad, Dn, Dv)
                 and not (self.inference_mode and isinstance(start_pos, torch.Tensor))):
             start = int(start_pos) if self.inference_mode else 0
-            if kernels.use_expanded(B, T, start, H, R, self.fp8_cache, self._cus(dev)):
-                o = self._expanded_attention(q, cache, cos, sin, B, T, start, rope_abs)
+            o = None
+            if x.dtype == torch.bfloat16:
+                if kernels.use_expanded(B, T, start, H, R, self.fp8_cache, self._cus(dev)):
+                    o = self._expanded_attention(q, cache, cos, sin, B, T, start, rope_abs)
+            elif (x.dtype == torch.float32 and not self.fp8_cache
+                  and kernels.use_expanded_f32(B, T, start, H, R, self._cus(dev))):
+                o = self._expanded_attention_f32(q, cache, cos, sin, B, T, start, rope_abs)
+            if o is not None:
                 return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
 
         n_splits, min_chunk, balance = self._decode_plan(

@@ -164,3 +164,68 @@ def test_prompt_in_a_graph(gpu):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("rope_abs", [False, True], ids=["chunk", "abs"])
+@pytest.mark.parametrize("B,T,start,H", [
+    (1, 1, 0, 1), (2, 2, 31, 3), (1, 31, 0, 2), (1, 32, 0, 2), (3, 33, 33, 1), (1, 64, 191, 2), (1, 257, 0, 16),
+    (2, 300, 700, 2),
+])
+def test_prompt_attention_f32(gpu, B, T, start, H, rope_abs):
+    """Edges of the 32-query blocks, the 32-token tiles and the eight waves
+    they are dealt to (fewer tiles than waves, one more than a round).  Every
+    product and sum is fp32: a score's error is at most about 200 roundings of
+    its terms (2^-24 each), a weight's twice that."""
+    say(f"prompt f32 B={B} T={T} start={start} H={H} rope_abs={rope_abs}")
+    g = torch.Generator(device=gpu).manual_seed(11 * T + start)
+    L, S = start + T, start + T + 3
+    cache = LatentCache.allocate(B, S, torch.float32, gpu, rank=64)
+    cache.kpe.copy_(torch.randn(B, S, 64, generator=g, device=gpu))
+    q = (0.8 * torch.randn(B * T, H, 196, generator=g, device=gpu))[:, :, :192]
+    kv = torch.randn(B, L, H, 256, generator=g, device=gpu)
+    cos, sin = (t[0, 0, :, :32].contiguous().to(gpu) for t in rope_tables(64, S))
+    out = torch.full((B * T, H, 132), 7.0, device=gpu)
+    kernels.prompt_attention_f32(q, cos, sin, kv, cache, SCALE, start=start, tokens_per_seq=T, rope_abs=rope_abs,
+                                 out=out[:, :, :128])
+    torch.cuda.synchronize()
+    qd = q.double().view(B, T, H, 192).transpose(1, 2)
+    r0 = start if rope_abs else 0
+    c, s = cos[r0:r0 + T].double(), sin[r0:r0 + T].double()
+    x1, x2 = qd[..., 128::2], qd[..., 129::2]
+    qd = torch.cat([qd[..., :128], torch.stack([x1 * c - x2 * s, x2 * c + x1 * s], -1).flatten(-2)], -1)
+    kd = torch.cat([kv[..., :128].transpose(1, 2), cache.kpe[:, None, :L].expand(B, H, L, 64)], -1).double()
+    mask = torch.arange(L, device=gpu)[None] > start + torch.arange(T, device=gpu)[:, None]
+    p = torch.softmax((qd @ kd.transpose(-1, -2) * SCALE).masked_fill(mask, float("-inf")), -1)
+    vd = kv[..., 128:].transpose(1, 2).double()
+    ref = p @ vd
+    e = 200 * 2.0 ** -24 * SCALE * (qd.abs() @ kd.abs().transpose(-1, -2)).amax(-1, keepdim=True)
+    bound = (p @ vd.abs()) * (2 * e + L * 2.0 ** -24)
+    got = out[:, :, :128].double().view(B, T, H, 128).transpose(1, 2)
+    assert bool(((got - ref).abs() <= bound).all()), float(((got - ref).abs() / bound).max())
+    assert bool((out[:, :, 128:] == 7.0).all())
+
+
+@pytest.mark.parametrize("rank,H", [(256, 16), (173, 12)])
+def test_module_f32_routes_agree(gpu, rank, H, monkeypatch):
+    """An fp32 prompt and a chunk behind it on either route: equal to fp32
+    sums in another order (1e-5 of the output's scale), cache bits equal."""
+    cfg = MLAConfig(n_embd=512, n_head=H, kv_lora_rank=rank, max_batch_size=2, max_seq_len=260)
+    m = MLA(cfg)
+    g = torch.Generator().manual_seed(rank)
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            if name.endswith("weight") and "norm" not in name:
+                p.copy_(torch.randn(p.shape, generator=g) * 0.03)
+    m.eval().to(gpu)
+    x0, x1 = (torch.randn(2, t, 512, generator=g).to(gpu) for t in (200, 45))
+    outs = {}
+    for use in (True, False):
+        monkeypatch.setattr(kernels, "use_expanded_f32", lambda *a, **k: use)
+        m.clear_cache()
+        m.set_inference_mode(True)
+        with torch.no_grad():
+            outs[use] = [m(x0, 0), m(x1, 200), m.kv_cache.clone()]
+    torch.cuda.synchronize()
+    for a, b in zip(outs[True], outs[False]):
+        assert float((a.double() - b.double()).abs().max()) <= 1e-5 * float(b.abs().max())
+    assert torch.equal(outs[True][2], outs[False][2])
