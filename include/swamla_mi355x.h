@@ -103,7 +103,7 @@ const char* mla_last_error(void);
  *              FP8); the LayerNorm covers the R channels, R.. are written 0.
  * kpe_cache    [cache_batch, cache_seq, P] in in_dtype.
  * ckv_scale    [cache_batch, cache_seq] fp32, written only for FP8 (else NULL).
- * err_flag     optional device int32; a token whose cache row / position /
+ * err_flag     optional int32 the device can write (device or pinned host memory); a token whose cache row / position /
  *              RoPE row lies outside the buffers is skipped and sets it to 1.
  *
  * Numerics: the LayerNorm is PyTorch's CPU LayerNorm op for op (fp32 Welford

@@ -198,7 +198,8 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle torch.cuda.current_stream(device).cuda_stream holds, without building the Stream object
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def split_count(L: int, n_splits: int, min_chunk: int) -> int:

@@ -106,6 +106,11 @@ class IncrementalDecoder:
         mask = None
         if t > 1:
             mask = torch.triu(torch.full((t, t), float("-inf"), device=idx.device), diagonal=1)
+            # built here, so each MLA can take it as verified (the check is a
+            # device comparison the host waits for, per layer)
+            key = MLA._mask_key(mask, t)
+            for m in self.mlas:
+                m._mask_ok = (key, mask)
         for blk in self.blocks:
             x = blk(x, start_pos, None, mask)
         x = tr.ln_f(x[:, -1:, :])

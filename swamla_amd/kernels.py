@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
-from typing import Optional
+from typing import Optional, Union
 
 import torch
 
@@ -31,20 +31,43 @@ def padded_rank(rank: int) -> int:
 
 
 def _need_gpu(*ts: Optional[torch.Tensor]) -> torch.device:
-    dev = None
+    first, idx = None, -1
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"swamla_amd kernels run on the GPU only; got a tensor on {t.device}"
             )
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} vs {t.device}")
-    assert dev is not None
-    return dev
+        if first is None:
+            first, idx = t, t.get_device()
+        elif t.get_device() != idx:
+            raise RuntimeError(f"tensors on different devices: {first.device} vs {t.device}")
+    assert first is not None
+    return first.device
+
+
+class HostFlag:
+    """An int32 in pinned host memory that kernels set through ``err_flag``
+    (the store crosses to the host only when a token is skipped) and the host
+    reads without a copy or an event.  A copy of its owner starts without one
+    (it is copied and unpickled as None)."""
+
+    def __init__(self):
+        self._t = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._v = ctypes.c_int32.from_address(self._t.data_ptr())
+
+    def data_ptr(self) -> int:
+        return self._t.data_ptr()
+
+    def is_set(self) -> bool:
+        return self._v.value != 0
+
+    def clear(self) -> None:
+        self._v.value = 0
+
+    def __reduce__(self):
+        return (type(None), ())
 
 
 def _i32(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -172,7 +195,7 @@ def append(
     start_pos: Optional[torch.Tensor] = None,
     tokens_per_seq: int = 1,
     rope_abs: bool = False,
-    err_flag: Optional[torch.Tensor] = None,
+    err_flag: Union[torch.Tensor, HostFlag, None] = None,
 ) -> None:
     """Fused kv_norm + RoPE(k_pe) + (e4m3) + scatter of ``kv`` rows.
 
@@ -313,7 +336,7 @@ class FusedAppend:
     ln_w: torch.Tensor
     ln_b: torch.Tensor
     eps: float
-    err_flag: Optional[torch.Tensor] = None
+    err_flag: Union[torch.Tensor, HostFlag, None] = None
 
 
 def decode_attention(
@@ -401,7 +424,7 @@ def decode_attention(
                 and ln_b.numel() in (rk, rp)):
             raise ValueError("LayerNorm weight / bias must be contiguous [R] or [R_pad]")
         ln_w, ln_b = pad_rank(ln_w.reshape(-1), rk), pad_rank(ln_b.reshape(-1), rk)
-        _need_gpu(kv, ln_w, ln_b, append.err_flag)
+        _need_gpu(kv, ln_w, ln_b, None if isinstance(append.err_flag, HostFlag) else append.err_flag)
         _abi.check(
             lib.mla_decode_attn_append(
                 kv.data_ptr(), kv.stride(0), ln_w.data_ptr(), ln_b.data_ptr(), float(append.eps),
@@ -715,6 +738,12 @@ def prompt_value_order(device=None) -> torch.Tensor:
     so that a lane of the kernel ends up with consecutive channels)."""
     p = torch.arange(128, device=device)
     return 64 * ((p >> 2) & 1) + 16 * (p >> 5) + 4 * ((p >> 3) & 3) + (p & 3)
+
+
+def to_prompt_value_order(w: torch.Tensor) -> torch.Tensor:
+    """w [H, 128, R] with its 128 rows in prompt_value_order."""
+    H, _, R = w.shape
+    return w.unflatten(1, (2, 4, 4, 4)).permute(0, 2, 3, 1, 4, 5).reshape(H, 128, R)
 
 
 def prompt_attention(

@@ -77,6 +77,22 @@ from .rope import RoPE
 RopeMode = str  # "chunk" (reference: positions 0..T-1 of the call) or "absolute"
 
 
+def _weight(lin: nn.Module) -> torch.Tensor:
+    """lin.weight, past nn.Module's attribute lookup where it is a plain parameter."""
+    w = lin._parameters.get("weight")
+    return lin.weight if w is None else w
+
+
+def _bias(lin: nn.Module) -> Optional[torch.Tensor]:
+    p = lin._parameters
+    return p["bias"] if "bias" in p else lin.bias
+
+
+def _versions(*ts: Optional[torch.Tensor]) -> tuple:
+    """What a derived weight is rebuilt on: storage, version, dtype and device of its sources."""
+    return tuple([None if t is None else (t.data_ptr(), t._version, t.dtype, t.device) for t in ts])
+
+
 class MLA(nn.Module):
     def __init__(self, config, cache_dtype: Optional[str] = None, rope_positions: Optional[str] = None):
         super().__init__()
@@ -141,12 +157,15 @@ class MLA(nn.Module):
         self._wo_packed = None  # (key, wo.weight packed for mla_linear_packed)
         self._padded_w = {}  # name -> (key, zero-padded copy to R_pad): kv_norm, wkv_a, W_uv
         self._workspace: Optional[DecodeWorkspace] = None
+        # row p: position p for every sequence of the cache (what an eager
+        # step's int start_pos becomes on the device, without a launch)
+        self._positions: Optional[torch.Tensor] = None
         self._num_cus: Optional[int] = None
         # Out-of-range appends: the kernels skip a token whose cache position
-        # or RoPE row is outside the tables and set this device flag; an eager
-        # call reads it back asynchronously (pinned copy + event) and the next
-        # eager call raises, as would mla.py:413's slice assignment.
-        self._err: Optional[list] = None  # [device flag int32[1], pinned host copy, event or None]
+        # or RoPE row is outside the tables and set this flag in pinned host
+        # memory; the next eager call that finds it raises, as would
+        # mla.py:413's slice assignment.
+        self._err: Optional[kernels.HostFlag] = None
         self._mask_ok = None  # (key, tensor) of the last mask verified as the prompt's causal mask
         # Split-KV plan of decode launches: "auto" balances the rows' splits
         # over the CUs on the device when positions come as a tensor (ragged
@@ -168,7 +187,7 @@ class MLA(nn.Module):
         return self.cache_dtype == "fp8_e4m3"
 
     def _param_like(self) -> torch.Tensor:
-        return self.wkv_a.weight
+        return _weight(self._modules["wkv_a"])
 
     def set_inference_mode(self, mode: bool = True) -> None:
         """mla.py:184-225: allocate (True) or delete (False) the latent cache."""
@@ -223,6 +242,7 @@ class MLA(nn.Module):
             setattr(self, name, None)
         self.inference_mode = False
         self._workspace = None
+        self._positions = None
 
     def _apply(self, fn, recurse=True):
         # The e4m3 scale stays fp32 whatever dtype the module is cast to; it
@@ -237,45 +257,26 @@ class MLA(nn.Module):
         return out
 
     # ------------------------------------------------------------ errors
-    def _err_flag(self, device) -> Optional[torch.Tensor]:
-        if self._err is None or self._err[0].device != device:
-            if self._capturing():  # created by an eager call only (a captured zero-fill would rerun)
-                return None
-            flag = torch.zeros(1, dtype=torch.int32, device=device)
-            self._err = [flag, torch.zeros(1, dtype=torch.int32, pin_memory=True), None]
-        return self._err[0]
+    def _err_flag(self) -> Optional[kernels.HostFlag]:
+        if self._err is None and not self._capturing():  # pinned memory is allocated by an eager call only
+            self._err = kernels.HostFlag()
+        return self._err
 
     @staticmethod
     def _capturing() -> bool:
         return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
 
-    def _raise_cache_error(self) -> None:
-        flag, host, _ = self._err
-        flag.zero_()
-        host.zero_()
-        self._err[2] = None
+    def _poll_cache_errors(self) -> None:
+        """Raise for a flag that an earlier call's kernels have set by now (no
+        synchronisation; skipped under graph capture)."""
+        err = self._err
+        if err is None or not err.is_set() or self._capturing():
+            return
+        err.clear()
         raise RuntimeError(
             "an earlier call appended a token outside the latent cache or the RoPE table "
             "(start_pos + seqlen > max_seq_len, a negative start_pos, or a batch row past max_batch_size); "
             "those tokens were not written (mla.py:413 raises for the same input)")
-
-    def _poll_cache_errors(self) -> None:
-        """Raise for a flag an earlier eager call left set, if its read-back
-        has landed (no synchronisation; skipped under graph capture)."""
-        if self._err is None or self._capturing():
-            return
-        ev = self._err[2]
-        if ev is not None and ev.query() and int(self._err[1][0]) != 0:
-            self._raise_cache_error()
-
-    def _read_back_cache_errors(self) -> None:
-        if self._err is None or self._capturing():
-            return
-        flag, host, _ = self._err
-        host.copy_(flag, non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record()
-        self._err[2] = ev
 
     def check_cache_errors(self) -> None:
         """Synchronising check: raise RuntimeError if any append since the
@@ -283,28 +284,25 @@ class MLA(nn.Module):
         from a captured HIP graph), and clear the flag."""
         if self._err is None:
             return
-        if int(self._err[0].item()) != 0:
-            self._raise_cache_error()
-        self._err[1].zero_()
-        self._err[2] = None
+        torch.cuda.current_stream(self._param_like().device).synchronize()
+        self._poll_cache_errors()
 
     def latent_cache(self) -> LatentCache:
         """The module's cache buffers as a kernel-level ``LatentCache``."""
         if self.kv_cache is None or self.pe_cache is None:
             raise RuntimeError("no latent cache: call set_inference_mode(True) first")
-        dt = self._param_like().dtype
-        if self.pe_cache.dtype != dt or (not self.fp8_cache and self.kv_cache.dtype != dt):
+        dt, kv, pe = self._param_like().dtype, self.kv_cache, self.pe_cache
+        if pe.dtype != dt or (not self.fp8_cache and kv.dtype != dt):
             raise RuntimeError(
-                f"cache dtype ({self.kv_cache.dtype}/{self.pe_cache.dtype}) does not match the "
+                f"cache dtype ({kv.dtype}/{pe.dtype}) does not match the "
                 f"parameters ({dt}); convert the module before set_inference_mode(True)"
             )
-        return LatentCache(self.kv_cache, self.pe_cache, self.kv_scale if self.fp8_cache else None,
-                           self.kv_lora_rank)
+        return LatentCache(kv, pe, self.kv_scale if self.fp8_cache else None, self.kv_lora_rank)
 
     @property
     def rank_pad(self) -> int:
         """Latent channels stored per token: kv_lora_rank rounded up to 64."""
-        return kernels.padded_rank(self.kv_lora_rank)
+        return -64 * (-self.kv_lora_rank // 64)
 
     def _padded(self, name: str, src: torch.Tensor, build) -> torch.Tensor:
         """A derived weight, rebuilt when ``src`` changes: ``build()`` pads it
@@ -326,10 +324,10 @@ class MLA(nn.Module):
         """kv_norm's weight and bias zero-padded to R_pad (the kernels read
         R_pad entries; the padding takes no part in the LayerNorm)."""
         R = self.kv_lora_rank
-        w = self._padded("kv_norm.weight", self.kv_norm.weight,
-                         lambda: kernels.pad_rank(self.kv_norm.weight.detach(), R))
-        b = self._padded("kv_norm.bias", self.kv_norm.bias,
-                         lambda: kernels.pad_rank(self.kv_norm.bias.detach(), R))
+        norm = self._modules["kv_norm"]
+        wn, bn = _weight(norm), _bias(norm)
+        w = self._padded("kv_norm.weight", wn, lambda: kernels.pad_rank(wn.detach(), R))
+        b = self._padded("kv_norm.bias", bn, lambda: kernels.pad_rank(bn.detach(), R))
         return w, b
 
     def _wkv_a_padded(self) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
@@ -353,10 +351,11 @@ class MLA(nn.Module):
         """W_uv [H, Dv, R_pad] for mla_merge_project: a view of wkv_b.weight,
         or its zero-padded copy."""
         H, Dn, Dv, R = self.n_heads, self.qk_nope_head_dim, self.v_head_dim, self.kv_lora_rank
-        view = lambda: self.wkv_b.weight.detach().view(H, Dn + Dv, R)[:, Dn:, :]
+        w = _weight(self._modules["wkv_b"])
+        view = lambda: w.detach().view(H, Dn + Dv, R).narrow(1, Dn, Dv)
         if self.rank_pad == R:
             return view()
-        return self._padded("w_uv", self.wkv_b.weight, lambda: kernels.pad_rank(view(), R))
+        return self._padded("w_uv", w, lambda: kernels.pad_rank(view(), R))
 
     def _w_uv_fused(self) -> torch.Tensor:
         """_w_uv() over the fused step's heads (zero for the padding heads)."""
@@ -386,13 +385,12 @@ class MLA(nn.Module):
         prompt_attention's order of value channels: what expands a cached
         latent into its heads' keys and values (mla.py:427-437)."""
         H, Dn, Dv, R = self.n_heads, self.qk_nope_head_dim, self.v_head_dim, self.kv_lora_rank
-        src = self.wkv_b.weight
+        src = _weight(self._modules["wkv_b"])
         view = lambda: src.detach().view(H, Dn + Dv, R)
         w_uk = view()[:, :Dn] if self.rank_pad == R else self._derived(
             "w_uk.expand", src, lambda: kernels.pad_rank(view()[:, :Dn], R))
-        w_uv = self._derived(
-            "w_uv.expand", src,
-            lambda: kernels.pad_rank(view()[:, Dn:].index_select(1, kernels.prompt_value_order(src.device)), R))
+        w_uv = self._derived("w_uv.expand", src,
+                             lambda: kernels.pad_rank(kernels.to_prompt_value_order(view()[:, Dn:]), R))
         return w_uk, w_uv
 
     # ------------------------------------------------------------- weights
@@ -418,8 +416,9 @@ class MLA(nn.Module):
         re-associating mla.py:427), q_pe and the wkv_a rows (mla.py:281-288,
         :307).  The absorbed block is formed in fp32 and rounded once to the
         model dtype; rebuilt when any source weight changes."""
-        ws = (self.wq.weight, self.wkv_a.weight, self.wkv_b.weight, self.wq.bias, self.wkv_a.bias)
-        key = tuple(None if t is None else (t.data_ptr(), t._version, t.dtype, t.device) for t in ws)
+        mods = self._modules
+        wq_, wkv_a_ = mods["wq"], mods["wkv_a"]
+        key = _versions(_weight(wq_), _weight(wkv_a_), _weight(mods["wkv_b"]), _bias(wq_), _bias(wkv_a_))
         if self._decode_w is None or self._decode_w[0] != key:
             H, Dn, R, rp = self.n_heads, self.qk_nope_head_dim, self.kv_lora_rank, self.rank_pad
             Hp = self._fused_heads() or H  # heads past H: zero rows (padding to a launch's 16 heads)
@@ -463,8 +462,7 @@ class MLA(nn.Module):
     def _packed_wo(self) -> Optional["kernels.PackedWeight"]:
         """_wo_fused() in mla_linear_packed's layout (None when its shape is
         not covered); rebuilt when the weight changes."""
-        w = self.wo.weight
-        key = (w.data_ptr(), w._version, w.dtype, w.device, self._fused_heads())
+        key = (_versions(_weight(self._modules["wo"])), self._fused_heads())
         if self._wo_packed is None or self._wo_packed[0] != key:
             wp = None
             wf = self._wo_fused()
@@ -522,7 +520,7 @@ class MLA(nn.Module):
         absorbed block formed in fp32, rounded once)."""
         ws = (self.wq_a.weight, self.wq_b.weight, self.wkv_a.weight, self.wkv_b.weight, self.wq_a.bias,
               self.wq_b.bias, self.wkv_a.bias)
-        key = tuple(None if t is None else (t.data_ptr(), t._version, t.dtype, t.device) for t in ws)
+        key = _versions(*ws)
         if self._decode_w is None or self._decode_w[0] != key:
             H, Dn, R, rp, ql = self.n_heads, self.qk_nope_head_dim, self.kv_lora_rank, self.rank_pad, self.q_lora_rank
             Hp = self._fused_heads() or H
@@ -558,7 +556,7 @@ class MLA(nn.Module):
         module at R_pad <= 256 (each wave serves both head groups from one
         stream of the cache), else 16."""
         if (self.n_heads == 32 and self.rank_pad <= 256
-                and self.wkv_a.weight.dtype == torch.bfloat16):
+                and self._param_like().dtype == torch.bfloat16):
             return 32
         return kernels.H
 
@@ -578,35 +576,27 @@ class MLA(nn.Module):
         32, in one launch), kv_lora_rank up to 512, at most 128 query rows and
         128-aligned model widths; a q low-rank module runs its query through
         two products with q_norm between them."""
-        wq = self.wq if self.q_lora_rank == 0 else self.wq_a
-        q_bias = (wq.bias is not None) if self.q_lora_rank == 0 else (
-            (self.wq_a.bias is not None) and (self.wq_b.bias is not None))
-        return (
-            self._fused_heads() is not None
-            and self.rank_pad <= kernels.MFMA_MAX_RANK
-            and x.dtype == torch.bfloat16
-            and wq.weight.dtype == torch.bfloat16
-            and 0 < n <= kernels.LINEAR_MAX_ROWS
-            and self.dim % 128 == 0
-            and (self.n_heads * self.v_head_dim) % 128 == 0
-            and q_bias == (self.wkv_a.bias is not None)
-            and self.v_head_dim == 128
-        )
+        if (x.dtype != torch.bfloat16 or not 0 < n <= kernels.LINEAR_MAX_ROWS or self.rank_pad > kernels.MFMA_MAX_RANK
+                or self.dim % 128 != 0 or self.v_head_dim != 128 or self._fused_heads() is None):
+            return False
+        mods = self._modules
+        wq = mods["wq"] if self.q_lora_rank == 0 else mods["wq_a"]
+        q_bias = _bias(wq) is not None
+        if self.q_lora_rank > 0:
+            q_bias = q_bias and _bias(mods["wq_b"]) is not None
+        return _weight(wq).dtype == torch.bfloat16 and q_bias == (_bias(mods["wkv_a"]) is not None)
 
     def _wide_step_ok(self, x: torch.Tensor, n: int) -> bool:
         """The decode step above rank 512: bf16 modules with up to 16 heads of
-        the built dimensions, at most 128 query rows."""
-        q_bias = ([self.wq.bias] if self.q_lora_rank == 0 else [self.wq_a.bias, self.wq_b.bias]) + [self.wkv_a.bias]
-        return (
-            self.rank_pad > kernels.MFMA_MAX_RANK
-            and self.n_heads <= kernels.H
-            and x.dtype == torch.bfloat16
-            and self.wkv_a.weight.dtype == torch.bfloat16
-            and 0 < n <= kernels.LINEAR_MAX_ROWS
-            and self.qk_nope_head_dim == 128
-            and self.v_head_dim == 128
-            and len({b is None for b in q_bias}) == 1
-        )
+        the built dimensions, at most 128 query rows and 128-aligned widths."""
+        if (self.rank_pad <= kernels.MFMA_MAX_RANK or x.dtype != torch.bfloat16
+                or not 0 < n <= kernels.LINEAR_MAX_ROWS or self.n_heads > kernels.H or self.dim % 128 != 0
+                or self.qk_nope_head_dim != 128 or self.v_head_dim != 128):
+            return False
+        mods = self._modules
+        qs = [mods["wq"]] if self.q_lora_rank == 0 else [mods["wq_a"], mods["wq_b"]]
+        bias = {_bias(m) is None for m in qs + [mods["wkv_a"]]}
+        return len(bias) == 1 and _weight(mods["wkv_a"]).dtype == torch.bfloat16
 
     def _wide_weights(self):
         """(weight, bias or None, packed copy or None) of [wq | wkv_a (R_pad +
@@ -616,7 +606,7 @@ class MLA(nn.Module):
         ws = [first.weight, self.wkv_a.weight, first.bias, self.wkv_a.bias]
         if self.q_lora_rank > 0:
             ws += [self.wq_b.weight, self.wq_b.bias]
-        key = tuple(None if t is None else (t.data_ptr(), t._version, t.dtype, t.device) for t in ws)
+        key = _versions(*ws)
         if self._decode_w is None or self._decode_w[0] != key:
             pk = lambda w: kernels.pack_weight(w) if kernels.packed_ok(1, w.shape[0], w.shape[1]) else None
             extra = (kernels.H - self.n_heads) * self.qk_head_dim
@@ -653,6 +643,11 @@ class MLA(nn.Module):
         return self._derived("w_uk_t.wide", self.wkv_b.weight,
                              lambda: torch.cat([w, w.new_zeros((kernels.H - H,) + tuple(w.shape[1:]))], 0))
 
+    def _dropped(self, out: torch.Tensor) -> torch.Tensor:
+        """resid_dropout (mla.py:495), whose call is skipped where it is the identity."""
+        drop = self._modules["resid_dropout"]
+        return drop(out) if drop.training or drop._forward_hooks or drop._forward_pre_hooks else out
+
     def _check_geometry(self) -> None:
         if (self.n_heads < 1 or self.qk_rope_head_dim != kernels.P
                 or not 1 <= self.kv_lora_rank <= kernels.MAX_RANK):
@@ -681,7 +676,7 @@ class MLA(nn.Module):
         ``split_plan`` overrides the choice."""
         if self.split_plan not in ("auto", "static", "balanced"):
             raise ValueError(f"split_plan must be 'auto', 'static' or 'balanced', got {self.split_plan!r}")
-        dt = dtype if dtype is not None else self.wkv_a.weight.dtype
+        dt = dtype if dtype is not None else self._param_like().dtype
         fused = dt == torch.bfloat16 and self.rank_pad <= kernels.MFMA_MAX_RANK
         bpc = kernels.decode_blocks_per_cu(dt, self.fp8_cache, self.kv_lora_rank, fused, device)
         n_splits, min_chunk = self._split_plan(n_rows, max_len, device, bpc)
@@ -736,7 +731,6 @@ class MLA(nn.Module):
             out = self._forward_kernels(x, start_pos)
             if self.advance_positions and not self._advance_folded:
                 start_pos.add_(x.size(1))
-        self._read_back_cache_errors()
         return out
 
     def _advance_target(self, start_pos, sp: torch.Tensor, T: int) -> Optional[torch.Tensor]:
@@ -753,7 +747,8 @@ class MLA(nn.Module):
     def _fused_output(self, o: torch.Tensor, start_pos, sp: torch.Tensor, B: int, T: int) -> torch.Tensor:
         """wo over the decode step's o [n, heads * Dv] (mla.py:490-495)."""
         n = B * T
-        wo_b = None if self.wo.bias is None else self.wo.bias.detach()
+        wo_b = _bias(self._modules["wo"])
+        wo_b = None if wo_b is None else wo_b.detach()
         wo_p = self._packed_wo()
         if wo_p is not None and kernels.packed_ok(n, wo_p.N, wo_p.K):
             adv = self._advance_target(start_pos, sp, T)
@@ -761,7 +756,11 @@ class MLA(nn.Module):
             self._advance_folded = adv is not None
         else:
             out = kernels.linear(o, self._wo_fused(), bias=wo_b).view(B, T, self.dim)
-        return self.resid_dropout(out)
+        return self._dropped(out)
+
+    @staticmethod
+    def _mask_key(mask: torch.Tensor, T: int) -> tuple:
+        return (mask.data_ptr(), mask.device, mask.dtype, tuple(mask.stride()), mask._version, T)
 
     def _is_causal_prompt_mask(self, mask: torch.Tensor, T: int, start_pos) -> bool:
         """True for the mask SWAMLAModel passes with a prompt
@@ -776,7 +775,7 @@ class MLA(nn.Module):
             return False
         # the verified tensor is kept alive with its key, so an equal pointer is
         # the same storage and an equal version means it was not written since
-        key = (mask.data_ptr(), mask.device, mask.dtype, tuple(mask.stride()), mask._version, T)
+        key = self._mask_key(mask, T)
         if self._mask_ok is not None and self._mask_ok[0] == key:
             return True
         if self._capturing():
@@ -806,8 +805,7 @@ class MLA(nn.Module):
             ln_w, ln_b = self.kv_norm_params()
             kernels.append(kv, cache, ln_w, ln_b, self.kv_norm.eps, cos, sin,
                            start_pos=sp, tokens_per_seq=T, rope_abs=self.rope_positions == "absolute",
-                           err_flag=self._err_flag(x.device))
-        self._read_back_cache_errors()
+                           err_flag=self._err_flag())
 
     def input_projections(self, x: torch.Tensor, need_q: bool = True) -> tuple[Optional[torch.Tensor], torch.Tensor]:
         """(q [B*T, H, 192] or None, kv [B*T, R_pad + P]): the wkv_a rows
@@ -858,7 +856,14 @@ class MLA(nn.Module):
         start_pos = int(start_pos)
         if start_pos < 0 or start_pos + T > cache.ckv.shape[1]:
             raise ValueError(f"start_pos {start_pos} + seqlen {T} exceeds max_seq_len {cache.ckv.shape[1]}")
-        return torch.full((B,), start_pos, dtype=torch.int32, device=device)
+        if T > 1 or self._capturing():  # a captured call owns what it reads
+            return torch.full((B,), start_pos, dtype=torch.int32, device=device)
+        rows, seq = cache.ckv.shape[:2]
+        tab = self._positions
+        if tab is None or tab.shape[0] < seq or tab.shape[1] < rows or tab.device != device:
+            tab = torch.arange(seq, dtype=torch.int32, device=device)[:, None].expand(seq, rows).contiguous()
+            self._positions = tab
+        return tab[start_pos, :B]
 
     # Keys and values of a prompt are expanded for as many sequences at a time
     # as fit this many bytes (at least one).
@@ -951,7 +956,7 @@ class MLA(nn.Module):
         # append first (their rows attend to each other's new tokens).
         fold_append = fused and T == 1
         ln_w, ln_b = self.kv_norm_params()
-        err = self._err_flag(dev)
+        err = self._err_flag()
         if not fold_append:
             kernels.append(kv, cache, ln_w, ln_b, self.kv_norm.eps, cos, sin,
                            start_pos=sp, tokens_per_seq=T, rope_abs=rope_abs, err_flag=err)
@@ -970,7 +975,7 @@ class MLA(nn.Module):
                   and kernels.use_expanded_f32(B, T, start, H, R, self._cus(dev))):
                 o = self._expanded_attention_f32(q, cache, cos, sin, B, T, start, rope_abs)
             if o is not None:
-                return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
+                return self._dropped(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
 
         n_splits, min_chunk, balance = self._decode_plan(
             n, max_len, dev, isinstance(start_pos, torch.Tensor) and self.inference_mode, dtype=x.dtype)
@@ -1064,4 +1069,4 @@ class MLA(nn.Module):
             kernels.head_product(o_lat[:, :H], self._w_uv(), out=o.view(n, H, Dv))
         else:
             o = torch.bmm(o_lat[:, :H].transpose(0, 1), w_uv_t).transpose(0, 1).reshape(n, H * Dv)  # [n, H*Dv]
-        return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
+        return self._dropped(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
