@@ -9,6 +9,7 @@ that is not on a ROCm device is an error.
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass
 from typing import Optional, Union
 
@@ -249,6 +250,28 @@ def plan_splits(n_rows: int, max_len: int, num_cus: int = 256, blocks_per_cu: in
     target = max(1, (num_cus * blocks_per_cu + n_rows - 1) // n_rows)
     by_len = max(1, (max_len + min_chunk - 1) // min_chunk)
     return int(max(1, min(target, by_len, 1024))), int(min_chunk)
+
+
+def min_chunk_for(dtype: torch.dtype, rank: int, max_len: int) -> int:
+    """Fewest tokens a split of a module's decode launch should take.
+
+    bf16 up to rank 512: 256 (less makes no difference at the sizes where it
+    could: 26.3 / 26.1 / 25.4 / 25.9 us per layer-step at 1 x 576 tokens with
+    256 / 128 / 64 / 32).
+    bf16 above rank 512: sqrt(2 L), within 32 .. 256.  A token of a split costs
+    about 0.06 us there (the four waves share every 16-token sub-tile and meet
+    once per sub-tile), a further split of a row 0.12 us in the merge.
+    Layer-steps at rank 640, us, 256 / 128 / 64 / 32: 1 x 576 48.9 / 41.5 / 38.8
+    / 37.3, 1 x 8000 50.6 / 46.9 / 50.6 / 64.8, 1 x 30000 61 / 70 / 70 / 70.
+    fp32: 16.  The VALU kernel takes 0.9 us per token of a split: 307 / 186 /
+    126 / 95 us at 1 x 576, 82 with 16; 311 / 195 / 142 / 142 at 1 x 16000, 142
+    with 16."""
+    if dtype == torch.float32:
+        return 16
+    if padded_rank(rank) <= MFMA_MAX_RANK:
+        return 256
+    c = math.isqrt(2 * max(int(max_len), 1))
+    return min(256, max(32, 16 * ((c + 8) // 16)))
 
 
 _BLOCKS_PER_CU: dict = {}
@@ -717,17 +740,18 @@ def use_expanded_f32(n_seq: int, tokens_per_seq: int, start: int, heads: int, ra
     3070, 1 x 256 at 2000 231 / 2252, 1 x 16 at 4000 299 / 321.  The expansion
     is a GEMM at about 47 TFLOP/s, a workgroup of the attention takes 5 us per
     eight tiles; the VALU kernel 3.5 ms per million pairs, and 0.8 us per token
-    of its longest split.  Head counts other than 16 come over from 512 tokens
-    on (1 x 512 at 12 heads 117 / 605); below, they stay on the 16-head
-    launches over padded heads that the tests of those modules count."""
+    of its longest split.  Head counts other than 16 come over past 320
+    tokens (1 x 512 at 12 heads 118 / 606); up to there they stay on the
+    16-head launches over padded heads that the tests of those modules count
+    (2 x 160 tokens)."""
     B, T, L = n_seq, tokens_per_seq, start + tokens_per_seq
-    if heads != H and B * T < 512:
+    if heads != H and B * T <= 320:
         return False
     rp = padded_rank(rank)
     pairs = B * (T * start + T * (T + 1) / 2) * 1e-6
     expand = 10 + 2.0 * B * L * heads * 256 * rp / 47e6
     attn = max(5 + 5 * -(-L // 256), pairs * heads * 640 / 60)
-    chunk = min(L, max(256, L / -(-num_cus // (B * T))))
+    chunk = min(L, max(16, L / -(-num_cus // (B * T))))
     latent = 25 + -(-heads // H) * rp / 256 * max(3500 * pairs, 0.8 * chunk)
     return expand + attn < latent
 

@@ -662,8 +662,10 @@ class MLA(nn.Module):
             self._num_cus = torch.cuda.get_device_properties(device).multi_processor_count
         return self._num_cus
 
-    def _split_plan(self, n_rows: int, max_len: int, device, blocks_per_cu: int = 1) -> tuple[int, int]:
-        return kernels.plan_splits(n_rows, max_len, num_cus=self._cus(device), blocks_per_cu=blocks_per_cu)
+    def _split_plan(self, n_rows: int, max_len: int, device, blocks_per_cu: int = 1,
+                    dtype: torch.dtype = torch.bfloat16) -> tuple[int, int]:
+        return kernels.plan_splits(n_rows, max_len, num_cus=self._cus(device), blocks_per_cu=blocks_per_cu,
+                                   min_chunk=kernels.min_chunk_for(dtype, self.kv_lora_rank, max_len))
 
     def _decode_plan(self, n_rows: int, max_len: int, device, per_row_positions: bool,
                      dtype: Optional[torch.dtype] = None) -> tuple[int, int, int]:
@@ -679,7 +681,7 @@ class MLA(nn.Module):
         dt = dtype if dtype is not None else self._param_like().dtype
         fused = dt == torch.bfloat16 and self.rank_pad <= kernels.MFMA_MAX_RANK
         bpc = kernels.decode_blocks_per_cu(dt, self.fp8_cache, self.kv_lora_rank, fused, device)
-        n_splits, min_chunk = self._split_plan(n_rows, max_len, device, bpc)
+        n_splits, min_chunk = self._split_plan(n_rows, max_len, device, bpc, dt)
         if self.split_plan == "balanced" or (self.split_plan == "auto" and per_row_positions):
             bal, cap = kernels.balanced_splits(n_rows, self._num_cus, bpc)
             if bal:

@@ -77,3 +77,16 @@ def test_committed_traffic_matches_the_current_kernel_source():
     for heads in (16, 32):
         got = bench.measured_traffic(32, 4224, "bf16", heads=heads)
         assert got is not None and got[0] > 87_000_000, (heads, got)
+
+
+def test_min_chunk_by_dtype_rank_and_length():
+    """The smallest split of a module's decode plan: fixed for bf16 up to rank
+    512 and for fp32, growing with sqrt(2 L) above rank 512."""
+    f = kernels.min_chunk_for
+    assert f(torch.bfloat16, 256, 100) == f(torch.bfloat16, 512, 100000) == 256
+    assert f(torch.float32, 256, 1) == f(torch.float32, 1024, 100000) == 16
+    wide = [f(torch.bfloat16, 640, n) for n in (0, 1, 576, 2000, 8000, 30000, 1 << 20)]
+    assert wide == [32, 32, 32, 64, 128, 240, 256]
+    m = MLA(MLAConfig(kv_lora_rank=640, max_batch_size=1, max_seq_len=64)).to(torch.bfloat16)
+    m._num_cus = 256
+    assert m._split_plan(1, 2000, torch.device("cpu")) == (32, 64)
