@@ -761,45 +761,70 @@ __global__ __launch_bounds__(kDecWaves * 64, 1) void mla_decode_dma(DecodeArgs a
 // ===========================================================================
 // The per-wave design above keeps a wave's O^T for all R_pad channels (4 NB
 // accumulators) and Q^T for R_pad + 64 in registers; past NB = 8 that no
-// longer fits.  Here the four waves of a workgroup share every sub-tile of
-// the split and divide the channels instead: wave w owns the 64-channel
-// blocks c = w, w + 4, w + 8, w + 12 (those below NB) and rope dimensions
-// 16 w .. 16 w + 15.  Per 16-token sub-tile a wave
-//   * streams its own channel blocks of the 16 latent rows (2 KB each, laid
-//     out as a one-block sub-tile of the kernel above, with the same 8-chunk
-//     swizzle) and its 32-byte slice of the 16 rope rows into its own LDS
-//     ring with global_load_lds_dwordx4; a wave with fewer blocks than the
-//     most loaded one re-reads its last block into the spare slot, so every
-//     wave issues kVm instructions per sub-tile and the waits stay fixed;
-//   * forms its partial S^T[16 tok x 16 heads] over its channels
+// longer fits.  Here the four waves of a workgroup share every token of the
+// split and divide the channels instead: wave w owns the 64-channel blocks
+// c = w, w + 4, w + 8, w + 12 (those below NB) and rope dimensions
+// 16 w .. 16 w + 15.  Per step of 32 tokens (two 16-token tiles) a wave
+//   * streams its own channel blocks of the 32 latent rows (4 KB each: two
+//     tiles, each laid out as a one-block sub-tile of the kernel above, with
+//     the same 8-chunk swizzle) and its 32-byte slice of the 32 rope rows
+//     into its own LDS ring with global_load_lds_dwordx4;
+//   * forms its partial S^T[32 tok x 16 heads] over its channels
 //     (mfma_f32_16x16x32_bf16) and rope slice (mfma_f32_16x16x16_bf16);
 //   * writes the partial to a double-buffered LDS exchange area, passes one
 //     barrier, and reads the four partials back, added in wave order, so
 //     every wave holds the same scores and runs the same online softmax;
-//   * accumulates O^T for its own channels (C^T read transposed from LDS).
+//   * accumulates O^T for its own channels (C^T read transposed from LDS),
+//     both tiles in one mfma_f32_16x16x32_bf16: the lane's k slots 0..3 are
+//     tile 0's tokens 4 g .. 4 g + 3, slots 4..7 tile 1's, in C^T and P^T
+//     alike.
 // Each wave then writes its own channels of o_lat or of the split's partial;
 // wave 0 writes the log-sum-exp.  Numerics are the kernel's above: bf16
 // weights in the product, o normalised by their sum, the LSE from the fp32
 // weights, per-op rounded q_pe RoPE, query channels >= R zeroed.
+//
+// One workgroup has the CU to itself (the ring and, for e4m3, the decoded
+// tiles fill LDS), so one wave per SIMD runs the whole chain: K reads, score
+// products, exchange, softmax, C^T products.  The chain's latency, not the
+// stream, is what a step costs, and a step of two tiles pays it once for 32
+// tokens; a deeper ring gains nothing (one tile a step, 3 / 4 / 5 buffers:
+// 43.4 / 43.3 / 44.3 us at 32 x 4096 tokens, rank 640).  Measured, one tile a
+// step -> two (both waves' spare DMAs dropped, whole-line partial stores,
+// e4m3 K decoded in registers): 42.8 -> 36.8 us at 32 x 4096, rank 640
+// (5.0 TB/s); 131 -> 114.5 at 128 x 4096 (6.45 TB/s, the stream's ceiling);
+// 52.4 -> 49.5 at rank 1024; e4m3 51.9 -> 45.3 at rank 1024, 168.7 -> 147 at
+// 128 x 4096, rank 900 (the decode's LDS traffic and VALU work bound it).
 namespace {
+constexpr int kWideTok = 2 * kSubTok;  // tokens of a step
 template <int C_DT, int NB>
 struct WideGeo {
   static constexpr int RP = 64 * NB;
-  static constexpr int NBW = (NB + kDecWaves - 1) / kDecWaves;  // channel blocks of the most loaded wave
-  static constexpr int kBlk = kSubTok * 128;                    // one 64-channel block of 16 bf16 rows
-  static constexpr int kBlkC = C_DT == 2 ? kSubTok * 64 : kBlk;  // ring bytes of a block (e4m3: codes)
-  static constexpr int kPe = 1024;                              // 16 rope slices of 32 B (+ 512 B re-read)
-  static constexpr int kSc = C_DT == 2 ? 256 : 0;               // e4m3: 4 copies of the 16 scales
-  static constexpr int kSub = NBW * kBlkC + kPe + kSc;          // a wave's ring bytes of one sub-tile
-  static constexpr int kVm = (C_DT == 2 ? NBW + 2 : 2 * NBW + 1);  // DMA instructions per sub-tile
-  static constexpr int kStage = C_DT == 2 ? NBW * kBlk : 0;     // e4m3: the wave's blocks decoded to bf16
-  static constexpr int NBUF = 3, kFill = 2, kCap = 2;
-  static constexpr int kXch = 2 * kDecWaves * 1024;             // two exchange buffers of 4 waves x 64 lanes x 16 B
-  static constexpr int kWave = NBUF * kSub + kStage;
-  static constexpr int kLds = kDecWaves * kWave + kXch;
-  static_assert(kLds <= kLdsMax, "LDS budget");
-  static_assert((kFill + 1) * kVm < 64, "vmcnt range");
+  static constexpr int NBW = (NB + kDecWaves - 1) / kDecWaves;    // channel blocks of the most loaded waves,
+  static constexpr int kFull = NB - kDecWaves * (NBW - 1);        // waves 0 .. kFull - 1; the others have one fewer
+  static constexpr int kTile = kSubTok * 128;                     // one 64-channel block of 16 bf16 rows
+  static constexpr int kBlkC = kWideTok * (C_DT == 2 ? 64 : 128);  // ring bytes of a block's 32 rows (e4m3: codes)
+  static constexpr int kPe = kWideTok * 32;                       // 32 rope slices of 32 B
+  static constexpr int kSc = C_DT == 2 ? 256 : 0;                 // e4m3: 2 copies of the 32 scales
+  static constexpr int kStep = NB * kBlkC + kDecWaves * (kPe + kSc);  // ring bytes of a step, all waves
+  static constexpr int kStage = C_DT == 2 ? NB * 2 * kTile : 0;   // e4m3: the blocks decoded to bf16
+  static constexpr int kXch = 2 * kDecWaves * 2048;               // two exchange buffers of 4 waves x 2 tiles x 1 KB
+  static constexpr int NBUF = cmin(3, (kLdsMax - kXch - kStage) / kStep), kFill = 2, kCap = NBUF - 1;
+  static constexpr int kLds = NBUF * kStep + kStage + kXch;
+  // DMA instructions of a step for a wave with n blocks
+  static constexpr int vm_of(int n) { return C_DT == 2 ? 2 * n + 2 : 4 * n + 1; }
+  static_assert(NBUF >= 2 && kLds <= kLdsMax, "LDS budget");
+  static_assert(NBUF * vm_of(NBW) < 64, "vmcnt range");
+  // the epilogue turns the wave's partial in its ring: 16 rows of 68 floats a block
+  static_assert(NBUF * (NBW * kBlkC + kPe + kSc) >= NBW * kH * 68 * 4, "the partial fits the wave's ring");
+  static_assert(NBUF * ((NBW - 1) * kBlkC + kPe + kSc) >= (NBW - 1) * kH * 68 * 4, "the partial fits the wave's ring");
+  // blocks of the waves before w
+  __device__ static __forceinline__ int blocks_before(int w) { return (NBW - 1) * w + min(w, kFull); }
 };
+
+// slot of 16-byte chunk c of an e4m3 block's 64-byte row: c ^ swc(row).  The K
+// operand reads 32 bytes of each of 16 rows, which lie 4 rows to a 256-byte
+// window: the XOR spreads rows 0..7 and 8..15 over the two halves of a row.
+__device__ __forceinline__ int swc(int row) { return (row >> 2) & 3; }
 
 __device__ __forceinline__ void ds_write16(uint32_t addr, f32x4_t v) {
   asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory");
@@ -838,7 +863,7 @@ __global__ __launch_bounds__(kDecWaves * 64, 1) void mla_decode_wide(DecodeArgs 
   const uint16_t* qa = static_cast<const uint16_t*>(a.q_abs) + r * a.qa_rs + n * a.qa_hs;
 #pragma unroll
   for (int i = 0; i < NBW; ++i) {
-    const int c = min(w + kDecWaves * i, NB - 1);  // a spare block re-reads a valid one (never used)
+    const int c = min(w + kDecWaves * i, NB - 1);  // past the wave's blocks: a valid one again (never used)
 #pragma unroll
     for (int s = 0; s < 2; ++s) vm_load<4>(qa + 64 * c + 32 * s + 8 * g, qraw[i][s]);
   }
@@ -863,75 +888,101 @@ __global__ __launch_bounds__(kDecWaves * 64, 1) void mla_decode_wide(DecodeArgs 
   const int t0 = split * rsp.chunk;  // a multiple of 16
   const int t1 = min(L, t0 + rsp.chunk);
   const int t_last = t1 > 0 ? t1 - 1 : 0;
-  const int n_sub = t1 > t0 ? (t1 - t0 + kSubTok - 1) / kSubTok : 0;
+  const int n_step = t1 > t0 ? (t1 - t0 + kWideTok - 1) / kWideTok : 0;
   const int64_t row0 = static_cast<int64_t>((b < 0 || b >= a.cache_b) ? 0 : b) * a.cache_s;
 
-  // ---- the wave's ring: per sub-tile NBW latent blocks, then the rope slices
-  lds_u8* const wave_lds = lds + w * G::kWave;
-  lds_u8* const xch = lds + kDecWaves * G::kWave;
+  // ---- the wave's LDS: its ring (per step its latent blocks, then the rope
+  // slices, then the e4m3 scales), its decoded blocks (e4m3), its exchange slot
+  const int nb_before = G::blocks_before(w);
+  lds_u8* const wave_lds = lds + NBUF * (nb_before * G::kBlkC + w * (G::kPe + G::kSc));
+  lds_u8* const stage_p = lds + NBUF * G::kStep + nb_before * (2 * G::kTile);  // e4m3 only
+  lds_u8* const xch = lds + NBUF * G::kStep + G::kStage;
   const uint8_t* const ckv = static_cast<const uint8_t*>(a.ckv);
   const uint8_t* const kpe = static_cast<const uint8_t*>(a.kpe);
-  // DMA lane offsets: latent instruction q of a block covers rows 8 q + lane / 8,
-  // slot lane % 8 holding chunk (lane % 8) ^ swz<1>(row); rope: row (lane / 2) % 16,
-  // half lane % 2 of the wave's 32 bytes (lanes 32 .. 63 re-read lanes 0 .. 31's)
-  int lat_row[2];
-  uint32_t lat_col[2];
+  constexpr int kLatRow = C_DT == 2 ? RP : 2 * RP;  // bytes of a latent cache row
+  constexpr int kLatQ = G::kBlkC / 1024;            // DMA instructions of a block
+  // DMA lane offsets from a step's first row: latent instruction q of a block
+  // covers (bf16) rows 8 q + lane / 8, slot lane % 8 holding chunk (lane % 8)
+  // ^ swz<1>(row % 16), or (e4m3 codes) rows 16 q + lane / 4, slot lane % 4
+  // of the block's 64 bytes holding chunk (lane % 4) ^ swc(row); rope: row
+  // lane / 2, half lane % 2 of the wave's 32 bytes.
+  int lat_row[kLatQ];
+  uint32_t lat_col[kLatQ];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    lat_row[q] = 8 * q + (lane >> 3);
-    lat_col[q] = 16 * ((lane & 7) ^ swz<1>(lat_row[q]));
+  for (int q = 0; q < kLatQ; ++q) {
+    lat_row[q] = C_DT == 2 ? 16 * q + (lane >> 2) : 8 * q + (lane >> 3);
+    lat_col[q] = C_DT == 2 ? 16 * ((lane & 3) ^ swc(lat_row[q])) : 16 * ((lane & 7) ^ swz<1>(lat_row[q] & 15));
   }
-  const int pe_row = (lane >> 1) & 15;
+  const int pe_row = lane >> 1;
   const uint32_t pe_col = 32 * w + 16 * (lane & 1);
-  auto issue = [&](int k) {
-    const int tb = t0 + kSubTok * k;
-    lds_u8* const dst = wave_lds + (k % NBUF) * G::kSub;
-#pragma unroll
-    for (int i = 0; i < NBW; ++i) {
-      const int c = min(w + kDecWaves * i, NB - 1);
-      if constexpr (C_DT == 2) {
-        // e4m3 codes as they lie: row lane / 4, bytes 16 (lane % 4) of the block's 64
-        const int tok = min(tb + (lane >> 2), t_last);
-        dma16(ckv + (row0 + tok) * RP + 64 * c + 16 * (lane & 3), dst + i * G::kBlkC);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int tok = min(tb + lat_row[q], t_last);
-          dma16(ckv + (row0 + tok) * (2 * RP) + 128 * c + lat_col[q], dst + i * G::kBlk + 1024 * q);
-        }
-      }
-    }
-    const int tok = min(tb + pe_row, t_last);
-    dma16(kpe + (row0 + tok) * (2 * kP) + pe_col, dst + NBW * G::kBlkC);
-    if constexpr (C_DT == 2) dma4(a.ckv_scale + row0 + min(tb + (lane & 15), t_last), dst + NBW * G::kBlkC + G::kPe);
-  };
-  issue(0);
-#pragma unroll
-  for (int k = 1; k < G::kFill; ++k) issue(k);  // past n_sub: re-reads the split's last row
 
-  // operand addresses within one block (the one-block layout of mla_decode_dma)
-  const int sw_n = swz<1>(n);
-  uint32_t qk_b[2];
+  // step k of a wave with NBK blocks into ring buffer k % NBUF: vm_of(NBK)
+  // instructions.  Rows past the split's end re-read its last row (in bounds).
+  auto issue = [&](auto nbk, int k) {
+    constexpr int NBK = decltype(nbk)::value;
+    const int tb = t0 + kWideTok * k;
+    lds_u8* const dst = wave_lds + (k % NBUF) * (NBK * G::kBlkC + G::kPe + G::kSc);
+    lds_u8* const dpe = dst + NBK * G::kBlkC;
+    if (tb + kWideTok - 1 <= t_last) {  // uniform: the whole step is in the split
+      const uint8_t* lb = ckv + (row0 + tb) * kLatRow + (C_DT == 2 ? 64 : 128) * w;
+      const uint8_t* pb = kpe + (row0 + tb) * (2 * kP);
 #pragma unroll
-  for (int s = 0; s < 2; ++s) qk_b[s] = n * 128 + 16 * ((4 * s + g) ^ sw_n);
-  const int pv_row = 4 * g + (n >> 2);
-  const int pv_sw = swz<1>(pv_row);
-  uint32_t pv_m[4];
+      for (int i = 0; i < NBK; ++i)
 #pragma unroll
-  for (int m = 0; m < 4; ++m) pv_m[m] = pv_row * 128 + 16 * ((2 * m + ((n & 3) >> 1)) ^ pv_sw) + 8 * (n & 1);
-  const uint32_t pe_rd = NBW * G::kBlkC + n * 32 + 8 * g;
-  lds_u8* const stage_p = wave_lds + NBUF * G::kSub;  // e4m3 only
-  const uint32_t stage = lds_off(stage_p);
-  const uint32_t xw = lds_off(xch) + 1024 * w + 16 * lane;  // this wave's exchange slot (buffer 0)
-  const uint32_t xr = lds_off(xch) + 16 * lane;             // wave v's slot: + 1024 v
+        for (int q = 0; q < kLatQ; ++q)
+          dma16(lb + (C_DT == 2 ? 64 : 128) * kDecWaves * i + static_cast<uint32_t>(lat_row[q] * kLatRow + lat_col[q]),
+                dst + i * G::kBlkC + 1024 * q);
+      dma16(pb + static_cast<uint32_t>(pe_row * (2 * kP) + pe_col), dpe);
+      if constexpr (C_DT == 2) dma4(a.ckv_scale + row0 + tb + (lane & 31), dpe + G::kPe);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < NBK; ++i)
+#pragma unroll
+      for (int q = 0; q < kLatQ; ++q)
+        dma16(ckv + (row0 + min(tb + lat_row[q], t_last)) * kLatRow + (C_DT == 2 ? 64 : 128) * (w + kDecWaves * i) +
+                  lat_col[q],
+              dst + i * G::kBlkC + 1024 * q);
+    dma16(kpe + (row0 + min(tb + pe_row, t_last)) * (2 * kP) + pe_col, dpe);
+    if constexpr (C_DT == 2) dma4(a.ckv_scale + row0 + min(tb + (lane & 31), t_last), dpe + G::kPe);
+  };
 
   f32x4_t oacc[4 * NBW];
 #pragma unroll
   for (int i = 0; i < 4 * NBW; ++i) oacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_part = 0.f, e_part = 0.f;
 
-  // queries (and everything else issued before the DMAs) have landed
-  wait_vm<G::kFill * G::kVm>();
+  // operand addresses within one tile (the one-block layout of mla_decode_dma)
+  const int sw_n = swz<1>(n);
+  uint32_t qk_b[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) qk_b[s] = n * 128 + 16 * ((4 * s + g) ^ sw_n);
+  uint32_t ck_b[2];  // e4m3: the K operand's 8 codes of a tile's row n
+#pragma unroll
+  for (int s = 0; s < 2; ++s) ck_b[s] = n * 64 + 16 * ((2 * s + (g >> 1)) ^ swc(n)) + 8 * (g & 1);
+  const int pv_row = 4 * g + (n >> 2);
+  const int pv_sw = swz<1>(pv_row);
+  uint32_t pv_m[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) pv_m[m] = pv_row * 128 + 16 * ((2 * m + ((n & 3) >> 1)) ^ pv_sw) + 8 * (n & 1);
+  const uint32_t stage = lds_off(stage_p);
+  const uint32_t xw = lds_off(xch) + 2048 * w + 16 * lane;  // this wave's exchange slot (buffer 0)
+  const uint32_t xr = lds_off(xch) + 16 * lane;             // wave v's slot: + 2048 v
+
+  // The ring fills at once (past n_step: re-reads the split's last row).
+  constexpr int kFewest = G::kFull == kDecWaves ? NBW : NBW - 1;  // blocks of the waves kFull ..
+  const bool full = G::kFull == kDecWaves || w < G::kFull;        // uniform in the wave
+#pragma unroll
+  for (int k = 0; k < G::kFill; ++k) {
+    if (full) issue(std::integral_constant<int, NBW>{}, k);
+    else issue(std::integral_constant<int, kFewest>{}, k);
+  }
+
+  // The queries (and everything else issued before the DMAs) have landed.  The
+  // wait and the releases stand ahead of the branch on the wave's block count:
+  // a value read on both sides of a branch may be copied at its head, and a
+  // copy of a register that a vm_load is still filling holds what was there.
+  wait_vm<G::kFill * G::vm_of(kFewest)>();
 #pragma unroll
   for (int i = 0; i < NBW; ++i)
 #pragma unroll
@@ -958,133 +1009,180 @@ __global__ __launch_bounds__(kDecWaves * 64, 1) void mla_decode_wide(DecodeArgs 
   }
   const s16x4_t qpe = __builtin_bit_cast(s16x4_t, make_uint2(qp[0], qp[1]));
 
-  for (int k = 0; k < n_sub; ++k) {  // uniform
-    if (k + G::kCap >= G::kFill && k + G::kCap < n_sub) issue(k + G::kCap);
-    wait_subtiles<G::kVm, NBUF>(max(G::kFill, min(n_sub, k + G::kCap + 1)) - (k + 1));
-    const int tb = t0 + kSubTok * k;
-    const uint32_t sb = lds_off(wave_lds + (k % NBUF) * G::kSub);
-    uint32_t lat = sb;  // the bf16 blocks the operand reads take
-    float4 scv = make_float4(1.f, 1.f, 1.f, 1.f);
-    if constexpr (C_DT == 2) {
-      // scales of the lane's tokens 4 g .. 4 g + 3, and the codes decoded into
-      // the staging tile in the bf16 ring layout (each lane: 8 codes -> one
-      // 16-byte chunk, two chunks per block)
-      u32x4v_t sc = ds_read16<0>(sb + NBW * G::kBlkC + G::kPe + 16 * g);
-      s16x4_t cv[NBW][2];
-      static_for<0, NBW>([&](auto iI) {
+  // The whole stream of a wave with NBK blocks (the waves of a workgroup meet
+  // at the barriers of their own copies of the loop: n_step is the same).
+  auto stream = [&](auto nbk) {
+    constexpr int NBK = decltype(nbk)::value;
+    constexpr int kVm = G::vm_of(NBK);
+    constexpr int kSub = NBK * G::kBlkC + G::kPe + G::kSc;
+    for (int k = 0; k < n_step; ++k) {  // uniform
+      if (k + G::kCap >= G::kFill && k + G::kCap < n_step) issue(nbk, k + G::kCap);
+      wait_subtiles<kVm, NBUF>(max(G::kFill, min(n_step, k + G::kCap + 1)) - (k + 1));
+      const int tb = t0 + kWideTok * k;
+      const uint32_t sb = lds_off(wave_lds + (k % NBUF) * kSub);
+      const uint32_t pe = sb + NBK * G::kBlkC;
+      uint32_t lat = sb;  // the bf16 blocks the operand reads take
+      f32x4_t scv[2] = {f32x4_t{1.f, 1.f, 1.f, 1.f}, f32x4_t{1.f, 1.f, 1.f, 1.f}};
+      u32x4v_t kr[2][NBK][2];
+      s16x4_t kp[2];
+      if constexpr (C_DT == 2) {
+        // scales of the lane's tokens 4 g .. 4 g + 3 of each tile
+        u32x4v_t sc[2];
+        sc[0] = ds_read16<G::kPe>(pe + 16 * g);
+        sc[1] = ds_read16<G::kPe + 64>(pe + 16 * g);
+        // The codes are read as the K operand wants them (row n, 8 channels
+        // from 32 s + 8 g), decoded in registers, and only the C^T operand's
+        // copy goes through the staging tiles (bf16 ring layout).
+        s16x4_t cv[2][NBK][2];
+        static_for<0, 2>([&](auto tI) {
+          constexpr int T = decltype(tI)::value;
+          static_for<0, NBK>([&](auto iI) {
+            constexpr int I = decltype(iI)::value;
+            cv[T][I][0] = ds_read8<I * G::kBlkC + 1024 * T>(sb + ck_b[0]);
+            cv[T][I][1] = ds_read8<I * G::kBlkC + 1024 * T>(sb + ck_b[1]);
+          });
+          kp[T] = ds_read8<512 * T>(pe + n * 32 + 8 * g);
+        });
+        lds_fence();
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          tie(sc[t]);
+          tie(kp[t]);
+          scv[t] = f32x4_t{u2f(sc[t].x), u2f(sc[t].y), u2f(sc[t].z), u2f(sc[t].w)};
+#pragma unroll
+          for (int i = 0; i < NBK; ++i)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+              tie(cv[t][i][s]);
+              const uint2 raw = __builtin_bit_cast(uint2, cv[t][i][s]);
+              const uint2 d0 = e4m3x4_to_bf16x4_hw(raw.x), d1 = e4m3x4_to_bf16x4_hw(raw.y);
+              kr[t][i][s] = u32x4v_t{d0.x, d0.y, d1.x, d1.y};
+              lds_st<u32x4v_t>(stage_p + (2 * i + t) * G::kTile + qk_b[s], kr[t][i][s]);
+            }
+        }
+        lat = stage;
+      } else {
+        static_for<0, 2>([&](auto tI) {
+          constexpr int T = decltype(tI)::value;
+          static_for<0, NBK>([&](auto iI) {
+            constexpr int I = decltype(iI)::value;
+            kr[T][I][0] = ds_read16<(2 * I + T) * G::kTile>(lat + qk_b[0]);
+            kr[T][I][1] = ds_read16<(2 * I + T) * G::kTile>(lat + qk_b[1]);
+          });
+          kp[T] = ds_read8<512 * T>(pe + n * 32 + 8 * g);
+        });
+        lds_fence();
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+          for (int i = 0; i < NBK; ++i) {
+            tie(kr[t][i][0]);
+            tie(kr[t][i][1]);
+          }
+          tie(kp[t]);
+        }
+      }
+      s16x4_t ctr[2][NBK][4];
+      static_for<0, NBK>([&](auto iI) {
         constexpr int I = decltype(iI)::value;
-        cv[I][0] = ds_read8<I * G::kBlkC>(sb + 8 * lane);
-        cv[I][1] = ds_read8<I * G::kBlkC + 512>(sb + 8 * lane);
+        static_for<0, 4>([&](auto mI) {
+          constexpr int M = decltype(mI)::value;
+          ctr[0][I][M] = ds_read_tr16<2 * I * G::kTile>(lat + pv_m[M]);
+          ctr[1][I][M] = ds_read_tr16<(2 * I + 1) * G::kTile>(lat + pv_m[M]);
+        });
+      });
+
+      // this wave's partial scores, then the exchange
+      f32x4_t sp[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int i = 0; i < NBK; ++i)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            sp[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[t][i][s]), qb[i][s], sp[t],
+                                                            0, 0, 0);
+      // The rope term has an accumulator of its own, added on the VALU: an
+      // mfma_f32_16x16x16 taking the 16x16x32 chain's result as its C operand
+      // got too few wait states on gfx950 and read the accumulator before the
+      // chain's last product had landed (the last channel block's scores were
+      // lost); the VALU adds also keep the inline-asm store below off a
+      // matrix-core result.
+      f32x4_t spe[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        spe[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(kp[t], qpe, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      // (e4m3: the token's scale multiplies the latent part, as in mla_decode_dma)
+      const uint32_t xo = 2048 * kDecWaves * (k & 1);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        ds_write16(xw + xo + 1024 * t,
+                   f32x4_t{scv[t][0] * sp[t][0] + spe[t][0], scv[t][1] * sp[t][1] + spe[t][1],
+                           scv[t][2] * sp[t][2] + spe[t][2], scv[t][3] * sp[t][3] + spe[t][3]});
+      lds_fence();  // the partial (and the C^T reads) are in LDS
+      __builtin_amdgcn_s_barrier();
+      u32x4v_t xv[2][kDecWaves];
+      static_for<0, kDecWaves>([&](auto vI) {
+        constexpr int V = decltype(vI)::value;
+        xv[0][V] = ds_read16<2048 * V>(xr + xo);
+        xv[1][V] = ds_read16<2048 * V + 1024>(xr + xo);
       });
       lds_fence();
-      tie(sc);
-      scv = make_float4(u2f(sc.x), u2f(sc.y), u2f(sc.z), u2f(sc.w));
+      float x[2][4];
+      float mt = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < NBW; ++i)
+      for (int t = 0; t < 2; ++t) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          tie(cv[i][q]);
-          const uint2 raw = __builtin_bit_cast(uint2, cv[i][q]);
-          const int o = 512 * q + 8 * lane;  // code offset in the block: row o / 64, chunk (o % 64) / 8
-          const int tt = o >> 6, c0 = (o & 63) >> 3;
-          const uint2 d0 = e4m3x4_to_bf16x4_hw(raw.x), d1 = e4m3x4_to_bf16x4_hw(raw.y);
-          lds_st16(stage_p + i * G::kBlk + tt * 128 + 16 * (c0 ^ swz<1>(tt)), make_uint4(d0.x, d0.y, d1.x, d1.y));
+        for (int v = 0; v < kDecWaves; ++v) tie(xv[t][v]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float sv = ((u2f(xv[t][0][i]) + u2f(xv[t][1][i])) + u2f(xv[t][2][i])) + u2f(xv[t][3][i]);
+          x[t][i] = tb + kSubTok * t + 4 * g + i < t1 ? sv * a.scale_log2 : -INFINITY;
+          mt = fmaxf(mt, x[t][i]);
         }
-      lat = stage;
-    }
-    u32x4v_t kr[NBW][2];
-    static_for<0, NBW>([&](auto iI) {
-      constexpr int I = decltype(iI)::value;
-      kr[I][0] = ds_read16<I * G::kBlk>(lat + qk_b[0]);
-      kr[I][1] = ds_read16<I * G::kBlk>(lat + qk_b[1]);
-    });
-    s16x4_t kp = ds_read8<0>(sb + pe_rd);
-    lds_fence();
-#pragma unroll
-    for (int i = 0; i < NBW; ++i) {
-      tie(kr[i][0]);
-      tie(kr[i][1]);
-    }
-    tie(kp);
-    s16x4_t ctr[NBW][4];
-    static_for<0, NBW>([&](auto iI) {
-      constexpr int I = decltype(iI)::value;
-      static_for<0, 4>([&](auto mI) {
-        constexpr int M = decltype(mI)::value;
-        ctr[I][M] = ds_read_tr16<I * G::kBlk>(lat + pv_m[M]);
-      });
-    });
-
-    // this wave's partial scores, then the exchange
-    f32x4_t sp = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < NBW; ++i)
-      if (w + kDecWaves * i < NB) {  // uniform
-        sp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[i][0]), qb[i][0], sp, 0, 0, 0);
-        sp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[i][1]), qb[i][1], sp, 0, 0, 0);
       }
-    // The rope term has an accumulator of its own, added on the VALU: an
-    // mfma_f32_16x16x16 taking the 16x16x32 chain's result as its C operand
-    // got too few wait states on gfx950 and read the accumulator before the
-    // chain's last product had landed (the last channel block's scores were
-    // lost); the VALU adds also keep the inline-asm store below off a
-    // matrix-core result.
-    const f32x4_t spe = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(kp, qpe, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    // (e4m3: the token's scale multiplies the latent part, as in mla_decode_dma)
-    const f32x4_t stot = f32x4_t{scv.x * sp[0] + spe[0], scv.y * sp[1] + spe[1], scv.z * sp[2] + spe[2],
-                                 scv.w * sp[3] + spe[3]};
-    const uint32_t xo = 4096 * (k & 1);
-    ds_write16(xw + xo, stot);
-    lds_fence();  // the partial (and the C^T reads) are in LDS
-    __builtin_amdgcn_s_barrier();
-    u32x4v_t xv[kDecWaves];
-    static_for<0, kDecWaves>([&](auto vI) {
-      constexpr int V = decltype(vI)::value;
-      xv[V] = ds_read16<1024 * V>(xr + xo);
-    });
-    lds_fence();
+      mt = wave_max_rows(mt);  // head n's maximum over the step (finite: token tb is valid)
+      if (__any(mt > m_run + kLazy)) {
+        const float m_new = fmaxf(m_run, mt);
+        const float alpha = exp2f(m_run - m_new);
+        m_run = m_new;
+        l_part *= alpha;
+        e_part *= alpha;
 #pragma unroll
-    for (int v = 0; v < kDecWaves; ++v) tie(xv[v]);
-    float x[4];
+        for (int i = 0; i < 4 * NBK; ++i) oacc[i] = oacc[i] * alpha;
+      }
+      uint32_t pw[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float sv = ((u2f(xv[0][i]) + u2f(xv[1][i])) + u2f(xv[2][i])) + u2f(xv[3][i]);
-      x[i] = tb + 4 * g + i < t1 ? sv * a.scale_log2 : -INFINITY;
+      for (int t = 0; t < 2; ++t) {
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = exp2f(x[t][i] - m_run);
+        const uint32_t w01 = pack_bf16x2(p[0], p[1]), w23 = pack_bf16x2(p[2], p[3]);
+        l_part += (u2f(w01 << 16) + u2f(w01 & 0xFFFF0000u)) + (u2f(w23 << 16) + u2f(w23 & 0xFFFF0000u));
+        e_part += (p[0] + p[1]) + (p[2] + p[3]);
+        pw[2 * t] = w01;
+        pw[2 * t + 1] = w23;
+        if constexpr (C_DT == 2) {
+          pw[2 * t] = pack_bf16x2(u2f(w01 << 16) * scv[t][0], u2f(w01 & 0xFFFF0000u) * scv[t][1]);
+          pw[2 * t + 1] = pack_bf16x2(u2f(w23 << 16) * scv[t][2], u2f(w23 & 0xFFFF0000u) * scv[t][3]);
+        }
+      }
+      const bf16x8_t pb = as_bf16x8(make_uint4(pw[0], pw[1], pw[2], pw[3]));
+#pragma unroll
+      for (int i = 0; i < NBK; ++i)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          tie(ctr[0][i][m]);
+          tie(ctr[1][i][m]);
+          const uint2 c0 = __builtin_bit_cast(uint2, ctr[0][i][m]), c1 = __builtin_bit_cast(uint2, ctr[1][i][m]);
+          oacc[4 * i + m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(make_uint4(c0.x, c0.y, c1.x, c1.y)), pb,
+                                                                    oacc[4 * i + m], 0, 0, 0);
+        }
     }
-    float mt = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-    mt = wave_max_rows(mt);  // head n's maximum over the sub-tile (finite: token tb is valid)
-    if (__any(mt > m_run + kLazy)) {
-      const float m_new = fmaxf(m_run, mt);
-      const float alpha = exp2f(m_run - m_new);
-      m_run = m_new;
-      l_part *= alpha;
-      e_part *= alpha;
-#pragma unroll
-      for (int i = 0; i < 4 * NBW; ++i) oacc[i] = oacc[i] * alpha;
-    }
-    float p[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] = exp2f(x[i] - m_run);
-    const uint32_t w01 = pack_bf16x2(p[0], p[1]), w23 = pack_bf16x2(p[2], p[3]);
-    l_part += (u2f(w01 << 16) + u2f(w01 & 0xFFFF0000u)) + (u2f(w23 << 16) + u2f(w23 & 0xFFFF0000u));
-    e_part += (p[0] + p[1]) + (p[2] + p[3]);
-    uint2 pw = make_uint2(w01, w23);
-    if constexpr (C_DT == 2) {
-      pw.x = pack_bf16x2(u2f(w01 << 16) * scv.x, u2f(w01 & 0xFFFF0000u) * scv.y);
-      pw.y = pack_bf16x2(u2f(w23 << 16) * scv.z, u2f(w23 & 0xFFFF0000u) * scv.w);
-    }
-    const s16x4_t pb = __builtin_bit_cast(s16x4_t, pw);
-#pragma unroll
-    for (int i = 0; i < NBW; ++i) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) tie(ctr[i][m]);
-      if (w + kDecWaves * i < NB)  // uniform
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-          oacc[4 * i + m] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ctr[i][m], pb, oacc[4 * i + m], 0, 0, 0);
-    }
-  }
-  wait_vm<0>();  // the ring's loads past the split's sub-tiles
+    wait_vm<0>();  // the ring's loads past the split's steps
+  };
+  if (full) stream(std::integral_constant<int, NBW>{});
+  else stream(std::integral_constant<int, kFewest>{});
 
   // ---- the wave's channels of head n: lane (n, g) holds O^T[16 m + 4 g + j][n]
   // of each block; l and e summed over the head's four lane groups
@@ -1111,19 +1209,30 @@ __global__ __launch_bounds__(kDecWaves * 64, 1) void mla_decode_wide(DecodeArgs 
     if (a.lse_out && w == 0 && g == 0) a.lse_out[static_cast<int64_t>(r) * kH + n] = lse2 * kLn2;
     return;
   }
-  const int64_t pidx = (static_cast<int64_t>(r) * a.n_splits + split) * kH + n;
-  float* op = a.o_part + pidx * RP + 4 * g;
+  // partials: each block turned through the wave's ring (free now) into 256
+  // contiguous bytes of a head per 16 lanes
+  const int64_t pidx = (static_cast<int64_t>(r) * a.n_splits + split) * kH;
+  constexpr int kTurn = 64 + 4;  // floats of a head's row
+  lds_u8* const turn = wave_lds;
+#pragma unroll
+  for (int i = 0; i < NBW; ++i)
+    if (w + kDecWaves * i < NB)
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        lds_st<f32x4_t>(turn + 4 * (kH * kTurn * i + kTurn * n + 16 * m + 4 * g), oacc[4 * i + m] * inv);
 #pragma unroll
   for (int i = 0; i < NBW; ++i) {
     const int c = w + kDecWaves * i;
     if (c < NB)
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
-        __builtin_nontemporal_store(f32x4_t{oacc[4 * i + m][0] * inv, oacc[4 * i + m][1] * inv,
-                                            oacc[4 * i + m][2] * inv, oacc[4 * i + m][3] * inv},
-                                    reinterpret_cast<f32x4_t*>(op + 64 * c + 16 * m));
+      for (int j = 0; j < 4; ++j) {
+        const int hd = 4 * j + g;
+        const f32x4_t v = *reinterpret_cast<__attribute__((address_space(3))) const f32x4_t*>(
+            turn + 4 * (kH * kTurn * i + kTurn * hd + 4 * n));
+        __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(a.o_part + (pidx + hd) * RP + 64 * c + 4 * n));
+      }
   }
-  if (w == 0 && g == 0) __builtin_nontemporal_store(lse2 * kLn2, a.lse_part + pidx);
+  if (w == 0 && g == 0) __builtin_nontemporal_store(lse2 * kLn2, a.lse_part + pidx + n);
 }
 
 // ===========================================================================

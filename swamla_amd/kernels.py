@@ -259,10 +259,10 @@ def min_chunk_for(dtype: torch.dtype, rank: int, max_len: int) -> int:
     could: 26.3 / 26.1 / 25.4 / 25.9 us per layer-step at 1 x 576 tokens with
     256 / 128 / 64 / 32).
     bf16 above rank 512: sqrt(2 L), within 32 .. 256.  A token of a split costs
-    about 0.06 us there (the four waves share every 16-token sub-tile and meet
-    once per sub-tile), a further split of a row 0.12 us in the merge.
-    Layer-steps at rank 640, us, 256 / 128 / 64 / 32: 1 x 576 48.9 / 41.5 / 38.8
-    / 37.3, 1 x 8000 50.6 / 46.9 / 50.6 / 64.8, 1 x 30000 61 / 70 / 70 / 70.
+    about 0.04 us there (the four waves share every 32-token step and meet
+    once per step), a further split of a row 0.12 us in the merge.
+    Layer-steps at rank 640, us, 256 / 128 / 64 / 32: 1 x 576 45.0 / 39.8 / 38.1
+    / 36.9, 1 x 8000 47.0 / 45.8 / 50.6 / 65.5, 1 x 30000 59 / 70 / 70 / 70.
     fp32: 16.  The VALU kernel takes 0.9 us per token of a split: 307 / 186 /
     126 / 95 us at 1 x 576, 82 with 16; 311 / 195 / 142 / 142 at 1 x 16000, 142
     with 16."""

@@ -87,3 +87,51 @@ def test_wide_step_equals_the_general_path(gpu, H, cache, q_lora, rank, monkeypa
     for a, b in zip(outs[True], outs[False]):
         err = (a.double() - b.double()).abs()
         assert not bool((err > 1e-2 + 2e-2 * b.double().abs()).any()), float(err.max())
+
+
+@pytest.mark.parametrize("rank", [513, 600, 704, 768, 832, 1024])
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "e4m3"])
+@pytest.mark.parametrize("n_splits,balance", [(1, 0), (5, 0), (40, 256)])
+def test_wide_attention_steps(gpu, rank, fp8, n_splits, balance):
+    """The channel-split attention against fp64 at the edges of its 32-token
+    steps and 16-token tiles, for every spread of channel blocks over the
+    waves (NB % 4 = 1, 2, 3, 0), launched three times.  A weight is rounded
+    to bf16 (2^-9, e4m3 again after the token's scale) and normalised by the
+    rounded weights' sum: within 3 x 2^-9 of the largest latent, plus the
+    output's own rounding (2^-9 of it); fp32 accumulation adds less than
+    2^-9 of the latent at these lengths."""
+    say(f"wide attention rank={rank} fp8={fp8} n_splits={n_splits}")
+    lens = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 95, 97, 129, 0, 513, 1000, 1999]
+    rows, S = len(lens), 2000
+    g = torch.Generator(device=gpu).manual_seed(rank + n_splits)
+    cache = LatentCache.allocate(rows, S, BF, gpu, fp8=fp8, rank=rank)
+    x = torch.randn(rows, S, rank, generator=g, device=gpu)
+    if fp8:
+        scale = x.abs().amax(-1) / 448
+        codes = (x / scale[..., None]).to(torch.float8_e4m3fn)
+        cache.ckv[..., :rank] = codes.view(torch.uint8)
+        cache.scale.copy_(scale)
+        lat = codes.double() * scale.double()[..., None]
+    else:
+        cache.ckv[..., :rank] = x.to(BF)
+        lat = cache.ckv[..., :rank].double()
+    cache.kpe.copy_(torch.randn(rows, S, 64, generator=g, device=gpu))
+    one, zero = torch.ones(S, 32, dtype=BF, device=gpu), torch.zeros(S, 32, dtype=BF, device=gpu)
+    rp = kernels.padded_rank(rank)
+    q_abs = (0.5 * torch.randn(rows, 16, rp, generator=g, device=gpu)).to(BF)
+    q_pe = torch.randn(rows, 16, 64, generator=g, device=gpu).to(BF)
+    sp = torch.tensor(lens, dtype=torch.int32, device=gpu) - 1
+    for _ in range(3):
+        lse = torch.empty(rows, 16, device=gpu)
+        o = kernels.decode_attention(q_abs, q_pe, one, zero, cache, 0.07, start_pos=sp, n_splits=n_splits,
+                                     min_chunk=16, lse_out=lse, balance=balance)
+        for r, n in enumerate(lens):
+            if n == 0:
+                assert bool((o[r] == 0).all()) and bool(torch.isneginf(lse[r]).all())
+                continue
+            s = 0.07 * (q_abs[r, :, :rank].double() @ lat[r, :n].T + q_pe[r].double() @ cache.kpe[r, :n].double().T)
+            ref = torch.softmax(s, -1) @ lat[r, :n]
+            lim = 2.0 ** -7 * float(lat[r, :n].abs().max()) + 2.0 ** -9 * ref.abs()
+            assert bool(((o[r, :, :rank].double() - ref).abs() <= lim).all()), (r, n)
+            assert float((lse[r].double() - torch.logsumexp(s, -1)).abs().max()) <= 1e-4, (r, n)
+            assert bool((o[r, :, rank:] == 0).all())
