@@ -65,6 +65,99 @@ constexpr int kPrKBytes = kPrTok * (kPrRow + kPrPe), kPrVBytes = kPrTok * kPrRow
 
 __device__ __forceinline__ int pr_swz(int t) { return ((t & 3) << 2) | ((t >> 2) & 3); }
 
+// One query row by one wave, tokens past its causal end never read.  The
+// kernels multiply a masked token's weight of 0 with its value; where that
+// value is not finite the product is NaN, and the rows that must not see the
+// token are computed again here (every row whose sums hold a NaN, so a row
+// that attends to one pays for this too).  A lane scores one token of 64 and
+// then sums two channels over them.
+template <bool F32>
+__device__ __forceinline__ void prompt_row(const PromptArgs& a, int b, int h, int t) {
+  using T = std::conditional_t<F32, float, uint16_t>;
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));  // nothing of this is computed ahead of the branch it stands in
+  auto val = [](T v) __attribute__((always_inline)) {
+    if constexpr (F32) return v;
+    else return bf16_to_f32(v);
+  };
+  const int Lq = a.start + t + 1;
+  const int64_t L = static_cast<int64_t>(a.start) + a.T;
+
+  // channels lane, 64 + lane and (rotated) 128 + lane of the query
+  const T* const qp = static_cast<const T*>(a.q) + (static_cast<int64_t>(b) * a.T + t) * a.q_rs + h * a.q_hs;
+  int rp = a.rope_abs ? a.start + t : t;
+  rp = rp >= a.rope_len ? static_cast<int>(a.rope_len) - 1 : rp;
+  const int64_t ro = static_cast<int64_t>(rp) * (kP / 2) + (lane >> 1);
+  const float cj = val(static_cast<const T*>(a.cos_tab)[ro]), sj = val(static_cast<const T*>(a.sin_tab)[ro]);
+  const float x1 = val(qp[kPrD + (lane & ~1)]), x2 = val(qp[kPrD + (lane | 1)]);
+  float qc[3] = {val(qp[lane]), val(qp[64 + lane]), 0.f};
+  if constexpr (F32) {
+    float u1, u2;
+    rope_pair<0>(x1, x2, cj, sj, u1, u2);
+    qc[2] = lane & 1 ? u2 : u1;
+  } else {
+    const uint32_t u = rope_bf16_packed(x1, x2, cj, sj);
+    qc[2] = bf16_to_f32(lane & 1 ? u >> 16 : u & 0xFFFF);
+  }
+
+  // rows of the keys and values: [B, H, L, 128] each, or (fp32) [B, L, H, 256]
+  const int64_t bh = static_cast<int64_t>(b) * a.H + h;
+  const int64_t row = F32 ? static_cast<int64_t>(a.H) * 2 * kPrD : kPrD;
+  const int64_t at = F32 ? (b * L * a.H + h) * 2 * kPrD : bh * L * kPrD;
+  const T* const kb = static_cast<const T*>(a.k) + at;
+  const T* const vb = F32 ? kb + kPrD : static_cast<const T*>(a.v) + at;
+  const T* const pe = static_cast<const T*>(a.kpe) + b * a.kpe_bs;
+  constexpr int kVec = 16 / sizeof(T);
+  float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll 1
+  for (int t0 = 0; t0 < Lq; t0 += 64) {
+    const int left = min(64, Lq - t0), tok = t0 + min(lane, left - 1);
+    float s = 0.f;
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      const T* const src = part < 2 ? kb + tok * row + 64 * part : pe + static_cast<int64_t>(tok) * kP;
+#pragma unroll 1
+      for (int c = 0; c < 64; c += kVec) {
+        T v[kVec];
+        __builtin_memcpy(v, __builtin_assume_aligned(src + c, 16), 16);
+#pragma unroll
+        for (int e = 0; e < kVec; ++e)
+          s = __builtin_fmaf(u2f(__builtin_amdgcn_readlane(f2u(qc[part]), c + e)), val(v[e]), s);
+      }
+    }
+    s = lane < left ? s * a.scale_log2 : -INFINITY;
+    float mt = s;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) mt = fmaxf(mt, shfl_xor_f32(mt, d));
+    const float m_new = fmaxf(m, mt);
+    const float alpha = m_new == m ? 1.f : __builtin_amdgcn_exp2f(m - m_new);  // both -inf: 1, not NaN
+    m = m_new;
+    float p = __builtin_amdgcn_exp2f(s - (m == -INFINITY ? 0.f : m));
+    if constexpr (!F32) p = bf16_to_f32(pack_bf16x2(p, 0.f) & 0xFFFF);
+    float sum = p;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) sum += shfl_xor_f32(sum, d);
+    l = l * alpha + sum;
+    o0 *= alpha, o1 *= alpha;
+#pragma unroll 1
+    for (int i = 0; i < left; ++i) {
+      const float w = u2f(__builtin_amdgcn_readlane(f2u(p), i));
+      const T* const v = vb + (t0 + i) * row + 2 * lane;
+      o0 = __builtin_fmaf(w, val(v[0]), o0);
+      o1 = __builtin_fmaf(w, val(v[1]), o1);
+    }
+  }
+  const float inv = 1.f / l;
+  T* const op = static_cast<T*>(a.out) + (static_cast<int64_t>(b) * a.T + t) * a.o_rs + h * a.o_hs;
+  if constexpr (F32) {
+    *reinterpret_cast<float2*>(op + 2 * lane) = make_float2(o0 * inv, o1 * inv);
+  } else {
+    const int pos = 2 * lane;  // position 32 c + 8 a + 4 f + e of a value row: channel 64 f + 16 c + 4 a + e
+    const int ch = 64 * ((pos >> 2) & 1) + 16 * (pos >> 5) + 4 * ((pos >> 3) & 3) + (pos & 3);
+    *reinterpret_cast<uint32_t*>(op + ch) = pack_bf16x2(o0 * inv, o1 * inv);
+  }
+}
+
 __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * (kPrKBytes + kPrVBytes)];
   const uint32_t lds_k = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)lds));
@@ -273,7 +366,16 @@ __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs
       stream(N{}, Y{}, 0, vbuf);
     }
   }
-  if (t_w + n >= a.T) return;  // surplus columns
+  if (w_tiles == 0) return;  // uniform: no query
+
+  // Columns whose sums hold a NaN (finite x 0 adds nothing): see prompt_row.
+  float nan_sum = 0.f;
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nan_sum = __builtin_fmaf(oacc[cb][r], 0.f, nan_sum);
+  const uint64_t bad2 = __ballot(t_w + n < a.T && nan_sum != 0.f);
+  uint32_t bad = static_cast<uint32_t>(bad2) | static_cast<uint32_t>(bad2 >> 32);
 
   // Lane (n, hf) holds positions 32 cb + 8 r4 + 4 hf + e of its query's
   // output; V's rows are laid out so that these are channels
@@ -282,16 +384,20 @@ __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs
   const float inv = 1.f / l_w;
   uint16_t* const op =
       static_cast<uint16_t*>(a.out) + (static_cast<int64_t>(b) * a.T + t_w + n) * a.o_rs + h * a.o_hs + 64 * hf;
+  if (t_w + n < a.T && !(bad >> n & 1)) {  // (surplus columns store nothing)
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb)
+    for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-    for (int r8 = 0; r8 < 2; ++r8) {
-      uint32_t o[4];
+      for (int r8 = 0; r8 < 2; ++r8) {
+        uint32_t o[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        o[e] = pack_bf16x2(oacc[cb][8 * r8 + 2 * e] * inv, oacc[cb][8 * r8 + 2 * e + 1] * inv);
-      *reinterpret_cast<uint4*>(op + 16 * cb + 8 * r8) = make_uint4(o[0], o[1], o[2], o[3]);
-    }
+        for (int e = 0; e < 4; ++e)
+          o[e] = pack_bf16x2(oacc[cb][8 * r8 + 2 * e] * inv, oacc[cb][8 * r8 + 2 * e + 1] * inv);
+        *reinterpret_cast<uint4*>(op + 16 * cb + 8 * r8) = make_uint4(o[0], o[1], o[2], o[3]);
+      }
+  }
+#pragma unroll 1
+  for (; bad != 0; bad &= bad - 1) prompt_row<false>(a, b, h, t_w + __builtin_ctz(bad));
 }
 
 // ---------------------------------------------------------------------------
@@ -443,7 +549,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void mla_prompt_f32_kernel(Prompt
   __syncthreads();
   for (int i = threadIdx.x; i < 32 * 32; i += kPfWaves * 64) {
     const int qi = i >> 5, c = 4 * (i & 31);
-    if (t0q + qi >= a.T) continue;
+    const bool live = t0q + qi < a.T;
     float m = -INFINITY;
     for (int k = 0; k < nw; ++k) m = fmaxf(m, m_lds[k][qi]);
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -456,8 +562,17 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void mla_prompt_f32_kernel(Prompt
       l += wk * l_lds[k][qi];
     }
     const float inv = 1.f / l;
-    *reinterpret_cast<float4*>(static_cast<float*>(a.out) + (static_cast<int64_t>(b) * a.T + t0q + qi) * a.o_rs +
-                               h * a.o_hs + c) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+    // a wave holds two rows, one per half: those with a NaN go to prompt_row
+    const uint64_t bad = __ballot(live && !(o.x * 0.f + o.y * 0.f + o.z * 0.f + o.w * 0.f == 0.f));
+    const bool half_bad = (hf ? bad >> 32 : bad & 0xFFFFFFFFu) != 0;
+    if (live && !half_bad)
+      *reinterpret_cast<float4*>(static_cast<float*>(a.out) + (static_cast<int64_t>(b) * a.T + t0q + qi) * a.o_rs +
+                                 h * a.o_hs + c) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+    if (bad != 0) {
+      const int q0 = t0q + __builtin_amdgcn_readfirstlane(qi);
+      if (bad & 0xFFFFFFFFu) prompt_row<true>(a, b, h, q0);
+      if (bad >> 32) prompt_row<true>(a, b, h, q0 + 1);
+    }
   }
 }
 

@@ -229,3 +229,58 @@ def test_module_f32_routes_agree(gpu, rank, H, monkeypatch):
     for a, b in zip(outs[True], outs[False]):
         assert float((a.double() - b.double()).abs().max()) <= 1e-5 * float(b.abs().max())
     assert torch.equal(outs[True][2], outs[False][2])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("where", ["v", "k", "pe"])
+@pytest.mark.parametrize("T,start,bad", [(200, 0, 1), (200, 0, 199), (65, 30, 40), (300, 100, 128), (40, 2, 31)])
+def test_later_nonfinite_tokens_stay_out(gpu, dtype, where, T, start, bad):
+    """A token's infinities and NaN reach the rows that attend to it and no
+    earlier one, at the edges of tiles and waves.  The clean rows are held to
+    the bounds of test_prompt_attention / test_prompt_attention_f32, in the
+    channels that hold no such value every row is."""
+    say(f"non-finite {where} {dtype} T={T} start={start} bad={bad}")
+    B, H = 2, 3
+    bf = dtype == torch.bfloat16
+    g = torch.Generator(device=gpu).manual_seed(T + bad)
+    L, S, tok = start + T, start + T + 3, start + bad
+    cache = LatentCache.allocate(B, S, dtype, gpu, rank=64)
+    cache.kpe.copy_(0.64 * torch.randn(B, S, 64, generator=g, device=gpu))
+    q = (0.8 * torch.randn(B * T, H, 192, generator=g, device=gpu)).to(dtype)
+    k, v = (torch.randn(B, H, L, 128, generator=g, device=gpu).to(dtype) for _ in range(2))
+    cos, sin = (t.to(dtype)[0, 0, :, :32].contiguous().to(gpu) for t in rope_tables(64, S))
+
+    qd = q.double().view(B, T, H, 192).transpose(1, 2)
+    c, s = cos[:T].double(), sin[:T].double()
+    x1, x2 = qd[..., 128::2], qd[..., 129::2]
+    qd = torch.cat([qd[..., :128], torch.stack([x1 * c - x2 * s, x2 * c + x1 * s], -1).flatten(-2)], -1)
+    kd = torch.cat([k, cache.kpe[:, None, :L].expand(B, H, L, 64)], -1).double()
+    mask = torch.arange(L, device=gpu)[None] > start + torch.arange(T, device=gpu)[:, None]
+    p = torch.softmax((qd @ kd.transpose(-1, -2) * SCALE).masked_fill(mask, float("-inf")), -1)
+    ref, spread = p @ v.double(), p @ v.double().abs()
+    if bf:
+        e = (3 * 2.0 ** -9 * SCALE * (qd[..., 128:].abs() @ kd[..., 128:].abs().transpose(-1, -2))).amax(-1, True)
+        bound = spread * (torch.expm1(2 * e) + 2 * 2.0 ** -9) + 2.0 ** -8 * ref.abs() + 1e-6
+    else:
+        e = 200 * 2.0 ** -24 * SCALE * (qd.abs() @ kd.abs().transpose(-1, -2)).amax(-1, True)
+        bound = spread * (2 * e + L * 2.0 ** -24)
+
+    hit = torch.zeros(B, H, T, 128, dtype=torch.bool, device=gpu)  # what the planted values may reach
+    if where == "v":
+        v[:, :, tok, 5::16] = float("inf")
+        v[:, :, L - 1, 6::16] = float("nan")
+        hit[:, :, bad:, 5::16] = True
+        hit[:, :, -1, 6::16] = True
+    else:
+        (k[:, :, tok] if where == "k" else cache.kpe[:, tok])[..., 3] = float("nan")
+        hit[:, :, bad:] = True
+    if bf:
+        out = kernels.prompt_attention(q, cos, sin, k, v[..., kernels.prompt_value_order(gpu)].contiguous(), cache,
+                                       SCALE, start=start, tokens_per_seq=T)
+    else:
+        out = kernels.prompt_attention_f32(q, cos, sin, torch.cat([k, v], -1).transpose(1, 2).contiguous(), cache,
+                                           SCALE, start=start, tokens_per_seq=T)
+    torch.cuda.synchronize()
+    got = out.double().view(B, T, H, 128).transpose(1, 2)
+    assert not bool(torch.isfinite(got[hit]).any())
+    assert bool(((got - ref).abs() <= bound)[~hit].all()), float(((got - ref).abs() - bound)[~hit].max())
