@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import weakref
 from dataclasses import dataclass
 from typing import Optional, Union
 
@@ -49,14 +50,39 @@ def _need_gpu(*ts: Optional[torch.Tensor]) -> torch.device:
 
 
 class HostFlag:
-    """An int32 in pinned host memory that kernels set through ``err_flag``
-    (the store crosses to the host only when a token is skipped) and the host
-    reads without a copy or an event.  A copy of its owner starts without one
-    (it is copied and unpickled as None)."""
+    """An int32 in pinned host memory that kernels on ``device`` set through
+    ``err_flag`` (the store crosses to the host only when a token is skipped)
+    and the host reads without a copy or an event.  A copy of its owner starts
+    without one (it is copied and unpickled as None).
 
-    def __init__(self):
+    Torch's pinned pool does not know which kernels hold the address, so a
+    dropped flag's memory is not returned to it while a store may be on its
+    way: it waits in ``_retired`` until the next flag is made, which first
+    waits for the devices of the flags it then lets go."""
+
+    _retired: list = []  # (tensor, device) of dropped flags
+
+    def __init__(self, device: torch.device):
+        self._release_retired()
+        self.device = device
         self._t = torch.zeros(1, dtype=torch.int32, pin_memory=True)
         self._v = ctypes.c_int32.from_address(self._t.data_ptr())
+        weakref.finalize(self, HostFlag._retired.append, (self._t, device)).atexit = False
+
+    @classmethod
+    def _release_retired(cls) -> None:
+        gone = []
+        while cls._retired:
+            try:
+                gone.append(cls._retired.pop())
+            except IndexError:  # another thread took it
+                break
+        try:
+            for dev in {d for _, d in gone}:
+                torch.cuda.synchronize(dev)
+        except BaseException:
+            cls._retired.extend(gone)
+            raise
 
     def data_ptr(self) -> int:
         return self._t.data_ptr()

@@ -257,9 +257,11 @@ class MLA(nn.Module):
         return out
 
     # ------------------------------------------------------------ errors
-    def _err_flag(self) -> Optional[kernels.HostFlag]:
-        if self._err is None and not self._capturing():  # pinned memory is allocated by an eager call only
-            self._err = kernels.HostFlag()
+    def _err_flag(self, device: torch.device) -> Optional[kernels.HostFlag]:
+        if self._err is None or self._err.device != device:
+            if self._capturing():  # pinned memory is allocated by an eager call only
+                return None
+            self._err = kernels.HostFlag(device)
         return self._err
 
     @staticmethod
@@ -284,7 +286,7 @@ class MLA(nn.Module):
         from a captured HIP graph), and clear the flag."""
         if self._err is None:
             return
-        torch.cuda.current_stream(self._param_like().device).synchronize()
+        torch.cuda.current_stream(self._err.device).synchronize()
         self._poll_cache_errors()
 
     def latent_cache(self) -> LatentCache:
@@ -807,7 +809,7 @@ class MLA(nn.Module):
             ln_w, ln_b = self.kv_norm_params()
             kernels.append(kv, cache, ln_w, ln_b, self.kv_norm.eps, cos, sin,
                            start_pos=sp, tokens_per_seq=T, rope_abs=self.rope_positions == "absolute",
-                           err_flag=self._err_flag())
+                           err_flag=self._err_flag(x.device))
 
     def input_projections(self, x: torch.Tensor, need_q: bool = True) -> tuple[Optional[torch.Tensor], torch.Tensor]:
         """(q [B*T, H, 192] or None, kv [B*T, R_pad + P]): the wkv_a rows
@@ -958,7 +960,7 @@ class MLA(nn.Module):
         # append first (their rows attend to each other's new tokens).
         fold_append = fused and T == 1
         ln_w, ln_b = self.kv_norm_params()
-        err = self._err_flag()
+        err = self._err_flag(dev)
         if not fold_append:
             kernels.append(kv, cache, ln_w, ln_b, self.kv_norm.eps, cos, sin,
                            start_pos=sp, tokens_per_seq=T, rope_abs=rope_abs, err_flag=err)
