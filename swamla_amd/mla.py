@@ -157,8 +157,10 @@ class MLA(nn.Module):
         self._wo_packed = None  # (key, wo.weight packed for mla_linear_packed)
         self._padded_w = {}  # name -> (key, zero-padded copy to R_pad): kv_norm, wkv_a, W_uv
         self._workspace: Optional[DecodeWorkspace] = None
-        # row p: position p for every sequence of the cache (what an eager
-        # step's int start_pos becomes on the device, without a launch)
+        # [max_seq_len, max_batch_size] int32, row p: position p for every
+        # sequence (what an eager step's int start_pos becomes on the device,
+        # without a launch).  Made and freed with the cache, 4 bytes beside
+        # each token's row, so that a step never writes it.
         self._positions: Optional[torch.Tensor] = None
         self._num_cus: Optional[int] = None
         # Out-of-range appends: the kernels skip a token whose cache position
@@ -229,10 +231,14 @@ class MLA(nn.Module):
                     ),
                     persistent=False,
                 )
+            rows, seq = self.kv_cache.shape[:2]
+            self._positions = torch.arange(seq, dtype=torch.int32, device=p.device)[:, None].expand(
+                seq, rows).contiguous()
         else:
             for name in ("k_cache", "v_cache", "kv_cache", "pe_cache", "kv_scale"):
                 if hasattr(self, name):
                     delattr(self, name)
+            self._positions = None
 
     def clear_cache(self) -> None:
         """mla.py:685-693, and leave inference mode so caches are reallocated."""
@@ -860,13 +866,12 @@ class MLA(nn.Module):
         start_pos = int(start_pos)
         if start_pos < 0 or start_pos + T > cache.ckv.shape[1]:
             raise ValueError(f"start_pos {start_pos} + seqlen {T} exceeds max_seq_len {cache.ckv.shape[1]}")
-        if T > 1 or self._capturing():  # a captured call owns what it reads
-            return torch.full((B,), start_pos, dtype=torch.int32, device=device)
-        rows, seq = cache.ckv.shape[:2]
         tab = self._positions
-        if tab is None or tab.shape[0] < seq or tab.shape[1] < rows or tab.device != device:
-            tab = torch.arange(seq, dtype=torch.int32, device=device)[:, None].expand(seq, rows).contiguous()
-            self._positions = tab
+        # a captured call owns what it reads; a cache put in place of the
+        # module's own, or moved with it, has no table
+        if (T > 1 or tab is None or tab.shape[0] < cache.ckv.shape[1] or tab.shape[1] < cache.ckv.shape[0]
+                or tab.device != device or self._capturing()):
+            return torch.full((B,), start_pos, dtype=torch.int32, device=device)
         return tab[start_pos, :B]
 
     # Keys and values of a prompt are expanded for as many sequences at a time
