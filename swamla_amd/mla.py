@@ -651,11 +651,6 @@ class MLA(nn.Module):
         return self._derived("w_uk_t.wide", self.wkv_b.weight,
                              lambda: torch.cat([w, w.new_zeros((kernels.H - H,) + tuple(w.shape[1:]))], 0))
 
-    def _dropped(self, out: torch.Tensor) -> torch.Tensor:
-        """resid_dropout (mla.py:495), whose call is skipped where it is the identity."""
-        drop = self._modules["resid_dropout"]
-        return drop(out) if drop.training or drop._forward_hooks or drop._forward_pre_hooks else out
-
     def _check_geometry(self) -> None:
         if (self.n_heads < 1 or self.qk_rope_head_dim != kernels.P
                 or not 1 <= self.kv_lora_rank <= kernels.MAX_RANK):
@@ -766,7 +761,7 @@ class MLA(nn.Module):
             self._advance_folded = adv is not None
         else:
             out = kernels.linear(o, self._wo_fused(), bias=wo_b).view(B, T, self.dim)
-        return self._dropped(out)
+        return self.resid_dropout(out)
 
     @staticmethod
     def _mask_key(mask: torch.Tensor, T: int) -> tuple:
@@ -984,7 +979,7 @@ class MLA(nn.Module):
                   and kernels.use_expanded_f32(B, T, start, H, R, self._cus(dev))):
                 o = self._expanded_attention_f32(q, cache, cos, sin, B, T, start, rope_abs)
             if o is not None:
-                return self._dropped(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
+                return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
 
         n_splits, min_chunk, balance = self._decode_plan(
             n, max_len, dev, isinstance(start_pos, torch.Tensor) and self.inference_mode, dtype=x.dtype)
@@ -1078,4 +1073,4 @@ class MLA(nn.Module):
             kernels.head_product(o_lat[:, :H], self._w_uv(), out=o.view(n, H, Dv))
         else:
             o = torch.bmm(o_lat[:, :H].transpose(0, 1), w_uv_t).transpose(0, 1).reshape(n, H * Dv)  # [n, H*Dv]
-        return self._dropped(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
+        return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
