@@ -88,6 +88,13 @@ def _bias(lin: nn.Module) -> Optional[torch.Tensor]:
     return p["bias"] if "bias" in p else lin.bias
 
 
+def _plain(m: nn.Module, cls: type) -> bool:
+    """Whether calling ``m`` is ``cls.forward`` on its parameters and nothing
+    else: no subclass or replacement, no forward of its own, no hooks."""
+    return (type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+            and not nn.modules.module._global_forward_hooks and not nn.modules.module._global_forward_pre_hooks)
+
+
 def _versions(*ts: Optional[torch.Tensor]) -> tuple:
     """What a derived weight is rebuilt on: storage, version, dtype and device of its sources."""
     return tuple([None if t is None else (t.data_ptr(), t._version, t.dtype, t.device) for t in ts])
@@ -596,15 +603,22 @@ class MLA(nn.Module):
 
     def _wide_step_ok(self, x: torch.Tensor, n: int) -> bool:
         """The decode step above rank 512: bf16 modules with up to 16 heads of
-        the built dimensions, at most 128 query rows and 128-aligned widths."""
-        if (self.rank_pad <= kernels.MFMA_MAX_RANK or x.dtype != torch.bfloat16
+        the built dimensions, at most 128 query rows and 128-aligned widths,
+        whose projections are plain layers (the general path calls them, so
+        that hooks and replacements act)."""
+        if (self.rank_pad <= kernels.MFMA_MAX_RANK or x.dtype != torch.bfloat16 or not x.is_cuda
                 or not 0 < n <= kernels.LINEAR_MAX_ROWS or self.n_heads > kernels.H or self.dim % 128 != 0
                 or self.qk_nope_head_dim != 128 or self.v_head_dim != 128):
             return False
         mods = self._modules
         qs = [mods["wq"]] if self.q_lora_rank == 0 else [mods["wq_a"], mods["wq_b"]]
-        bias = {_bias(m) is None for m in qs + [mods["wkv_a"]]}
-        return len(bias) == 1 and _weight(mods["wkv_a"]).dtype == torch.bfloat16
+        ins = qs + [mods["wkv_a"]]
+        if not all([_plain(m, nn.Linear) for m in ins + [mods["wo"]]]):
+            return False
+        if self.q_lora_rank > 0 and not _plain(mods["q_norm"], nn.LayerNorm):
+            return False
+        bias = {_bias(m) is None for m in ins}
+        return len(bias) == 1 and all([_weight(m).dtype == torch.bfloat16 for m in ins + [mods["wo"]]])
 
     def _wide_weights(self):
         """(weight, bias or None, packed copy or None) of [wq | wkv_a (R_pad +

@@ -416,6 +416,16 @@ def test_no_cpu_fallback():
         m(torch.randn(1, 1, 128), 0)
 
 
+def test_wide_projections_on_the_cpu():
+    """input_projections of a bf16 module above rank 512 takes CPU tensors (no
+    kernel is needed for them)."""
+    m = MLA(small_cfg(n_embd=512, kv_lora_rank=640)).to(torch.bfloat16)
+    x = torch.randn(1, 1, 512).to(torch.bfloat16)
+    with torch.no_grad():
+        q, kv = m.input_projections(x)
+        assert torch.equal(kv, m.wkv_a(x).view(1, -1)) and torch.equal(q.reshape(1, -1), m.wq(x).view(1, -1))
+
+
 def test_unsupported_paths_raise():
     m = MLA(small_cfg()).eval()
     x = torch.randn(1, 2, 128)

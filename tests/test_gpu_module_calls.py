@@ -60,3 +60,43 @@ def test_resid_dropout_is_called(gpu, rank, T, dtype):
         got = m(x, 0)
     torch.cuda.synchronize()
     assert torch.equal(got, 0.5 * want)
+
+
+@pytest.mark.parametrize("q_lora", [0, 160])
+def test_wide_step_calls_hooked_and_replaced_layers(gpu, q_lora, monkeypatch):
+    """Above rank 512 a decode step's projections may be wrapped: hooks on
+    them run, and a layer of another class with a weight of its own keeps its
+    own forward.  Plain layers take the step's own launches."""
+    say(f"wide step, hooks and replacements, q_lora={q_lora}")
+    m, x = layer(gpu, 2, kv_lora_rank=640, q_lora_rank=q_lora), hidden(gpu, 3, 1)
+    launches = []
+    real = kernels.merge_project_wide
+    monkeypatch.setattr(kernels, "merge_project_wide", lambda *a, **k: (launches.append(1), real(*a, **k))[1])
+    names = ["wkv_a", "wo"] + (["wq"] if q_lora == 0 else ["wq_a", "q_norm", "wq_b"])
+    with torch.no_grad():
+        m.prefill_cache(hidden(gpu, 3, 50), 0)
+        want = m(x, 50)
+        assert len(launches) == 1
+        for name in names:
+            seen = []
+            lin = getattr(m, name)
+            for register in (lin.register_forward_hook, lin.register_forward_pre_hook):
+                handle = register(lambda mod, *a: seen.append(mod))
+                got = m(x, 50)
+                handle.remove()
+                assert seen == [lin], name
+                seen.clear()
+            err = (got.double() - want.double()).abs()
+            assert not bool((err > 1e-2 + 2e-2 * want.double().abs()).any()), name
+
+        class Doubled(type(m.wo)):
+            def forward(self, x):
+                return 2 * super().forward(x)
+
+        plain, m.wo = m.wo, Doubled(*reversed(m.wo.weight.shape), bias=False).to(BF).to(gpu)
+        m.wo.load_state_dict(plain.state_dict())
+        err = (m(x, 50).double() - 2 * want.double()).abs()
+        assert not bool((err > 2e-2 + 2e-2 * 2 * want.double().abs()).any())
+        m.wo = plain
+        launches.clear()
+        assert torch.equal(m(x, 50), want) and len(launches) == 1
