@@ -319,6 +319,14 @@ class MLA(nn.Module):
         """Latent channels stored per token: kv_lora_rank rounded up to 64."""
         return -64 * (-self.kv_lora_rank // 64)
 
+    def _operand(self, name: str, w: torch.Tensor, src: torch.Tensor) -> torch.Tensor:
+        """``w``, a view of the parameter ``src``, or a copy of it where the
+        kernels' 16-byte loads need one (a parameter inside a flat buffer may
+        start anywhere; the copy is kept until ``src`` changes)."""
+        if w.data_ptr() % 16 == 0 and w.stride(-1) == 1 and w.stride(-2) % 8 == 0:
+            return w
+        return self._derived(name + ".operand", src, lambda: w.clone(memory_format=torch.contiguous_format))
+
     def _padded(self, name: str, src: torch.Tensor, build) -> torch.Tensor:
         """A derived weight, rebuilt when ``src`` changes: ``build()`` pads it
         to R_pad; ``src`` itself is used when kv_lora_rank needs no padding."""
@@ -369,7 +377,7 @@ class MLA(nn.Module):
         w = _weight(self._modules["wkv_b"])
         view = lambda: w.detach().view(H, Dn + Dv, R).narrow(1, Dn, Dv)
         if self.rank_pad == R:
-            return view()
+            return self._operand("w_uv", view(), w)
         return self._padded("w_uv", w, lambda: kernels.pad_rank(view(), R))
 
     def _w_uv_fused(self) -> torch.Tensor:
@@ -402,7 +410,7 @@ class MLA(nn.Module):
         H, Dn, Dv, R = self.n_heads, self.qk_nope_head_dim, self.v_head_dim, self.kv_lora_rank
         src = _weight(self._modules["wkv_b"])
         view = lambda: src.detach().view(H, Dn + Dv, R)
-        w_uk = view()[:, :Dn] if self.rank_pad == R else self._derived(
+        w_uk = self._operand("w_uk", view()[:, :Dn], src) if self.rank_pad == R else self._derived(
             "w_uk.expand", src, lambda: kernels.pad_rank(view()[:, :Dn], R))
         w_uv = self._derived("w_uv.expand", src,
                              lambda: kernels.pad_rank(kernels.to_prompt_value_order(view()[:, Dn:]), R))
@@ -468,9 +476,9 @@ class MLA(nn.Module):
         zero columns for the padding heads (whose read-out is zero)."""
         H, Dv = self.n_heads, self.v_head_dim
         Hp = self._fused_heads() or H
-        if Hp == H:
-            return self.wo.weight.detach()
         w = self.wo.weight.detach()
+        if Hp == H:
+            return self._operand("wo", w, self.wo.weight)
         return self._derived("wo.weight.fused", self.wo.weight,
                              lambda: torch.cat([w, w.new_zeros(w.shape[0], (Hp - H) * Dv)], 1))
 
@@ -515,15 +523,17 @@ class MLA(nn.Module):
                  wp: Optional["kernels.PackedWeight"]) -> torch.Tensor:
         """x . w^T (+ b) for the decode step: mla_linear_packed with the packed
         copy while its grid fits the CUs in one round; past that, or for a K
-        the kernels do not take, the library GEMM; else mla_linear."""
+        or N the kernels do not take, the library GEMM; else mla_linear."""
         n, K = x.shape
+        if x.data_ptr() % 16 != 0 or x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < K:
+            x = x.clone(memory_format=torch.contiguous_format)  # rows as the kernels' 16-byte loads need them
         if wp is not None and kernels.packed_ok(n, wp.N, wp.K):
             if self._num_cus is None:
                 self._num_cus = torch.cuda.get_device_properties(x.device).multi_processor_count
             if kernels.packed_blocks(n, wp.N, wp.K) <= self._num_cus:
                 return kernels.linear_packed(x, wp, bias=b)
             return torch.nn.functional.linear(x, w, b)
-        if K % 128 == 0 and x.stride(1) == 1:
+        if K % 128 == 0 and w.shape[0] % 16 == 0:
             return kernels.linear(x, w, bias=b)
         return torch.nn.functional.linear(x, w, b)
 
@@ -653,8 +663,8 @@ class MLA(nn.Module):
         nq = sets[0][0].shape[0] - (self.rank_pad + self.qk_rope_head_dim)
         q = y[:, :nq]
         if self.q_lora_rank > 0:
-            q = torch.nn.functional.layer_norm(q, (nq,), self.q_norm.weight, self.q_norm.bias, self.q_norm.eps)
-            q = self._product(q, *sets[1])
+            qn = torch.nn.functional.layer_norm(q, (nq,), self.q_norm.weight, self.q_norm.bias, self.q_norm.eps)
+            q = self._product(qn.to(q.dtype), *sets[1])  # (autocast normalises in fp32)
         return q.view(n, kernels.H, self.qk_head_dim), y[:, nq:]
 
     def _w_uk_t_wide(self) -> torch.Tensor:
