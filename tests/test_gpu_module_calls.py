@@ -102,44 +102,43 @@ def test_wide_step_calls_hooked_and_replaced_layers(gpu, q_lora, monkeypatch):
         assert torch.equal(m(x, 50), want) and len(launches) == 1
 
 
-def misplace(m):
-    """Every parameter moved into one flat buffer, 2-byte aligned only."""
-    ps = list(m.parameters())
+def misplace(m, names):
+    """Parameters moved into one flat buffer, 2-byte aligned only."""
+    ps = [p for n, p in m.named_parameters() if n.startswith(names)]
     buf = torch.empty(sum(p.numel() + 9 for p in ps), dtype=ps[0].dtype, device=ps[0].device)
     at = 1
     for p in ps:
         view = buf[at:at + p.numel()].view(p.shape)
         view.copy_(p.data)
         p.data = view
-        at += p.numel() + (9 if (at + p.numel()) % 8 == 0 else 8 - (at + p.numel()) % 8 + 1)
-    assert all(p.data_ptr() % 16 == 2 for p in ps)
+        at += p.numel()
+        at += 1 + -at % 8
+    assert ps and all(p.data_ptr() % 16 == 2 for p in ps)
 
 
 @pytest.mark.parametrize("rank,q_lora,heads", [(640, 0, 16), (640, 100, 16), (640, 128, 12), (1000, 160, 16)])
 @pytest.mark.parametrize("T", [1, 300])
 def test_parameters_and_inputs_in_any_layout(gpu, rank, q_lora, heads, T):
     """Above rank 512, where steps and prompts were ATen products that take
-    any layout: parameters at odd addresses, a q_lora_rank the kernels' widths
-    do not divide, and inputs that are misaligned, expanded or transposed
-    views give what aligned ones give."""
+    any layout: parameters at odd addresses (a prompt's own GEMMs keep
+    aligned ones: only wkv_b is moved), a q_lora_rank the kernels' widths do
+    not divide, and inputs that are misaligned, expanded or transposed views
+    give what aligned ones give."""
     say(f"layouts rank={rank} q_lora={q_lora} heads={heads} T={T}")
     m = layer(gpu, 3, kv_lora_rank=rank, q_lora_rank=q_lora, n_head=heads)
     x, start = hidden(gpu, 2, T), 40 if T == 1 else 0
 
-    def same(got, want):  # a prompt's GEMMs may be other ones for another layout
-        bar = 0 if T == 1 else 1e-2 + 2e-2 * want.double().abs()
-        assert bool(((got.double() - want.double()).abs() <= bar).all())
-
     with torch.no_grad():
         m.prefill_cache(hidden(gpu, 2, 40), 0)
         want = m(x, start)
-        wide = torch.zeros(2, T, 515, dtype=BF, device=gpu)
-        wide[:, :, 3:] = x
-        same(m(wide[:, :, 3:], start), want)
-        same(m(x.transpose(0, 2).contiguous().transpose(0, 2), start), want)
-        same(m(x[:1].expand(2, T, 512), start), m(x[:1].repeat(2, 1, 1), start))
-        misplace(m)
-        same(m(x, start), want)
+        if T == 1:
+            wide = torch.zeros(2, T, 515, dtype=BF, device=gpu)
+            wide[:, :, 3:] = x
+            assert torch.equal(m(wide[:, :, 3:], start), want)
+        assert torch.equal(m(x.transpose(0, 2).contiguous().transpose(0, 2), start), want)
+        assert torch.equal(m(x[:1].expand(2, T, 512), start), m(x[:1].repeat(2, 1, 1), start))
+        misplace(m, ("w", "q_norm", "kv_norm") if T == 1 else ("wkv_b",))
+        assert torch.equal(m(x, start), want)
         if q_lora and T == 1:
             with torch.autocast("cuda", dtype=BF):
                 got = m(x, start)
