@@ -893,52 +893,68 @@ class MLA(nn.Module):
             return torch.full((B,), start_pos, dtype=torch.int32, device=device)
         return tab[start_pos, :B]
 
-    # Keys and values of a prompt are expanded for as many sequences at a time
-    # as fit this many bytes (at least one).
+    # Keys and values of a prompt take at most this many bytes at a time.
     EXPAND_BYTES = 512 << 20
 
+    def _expand_groups(self, B: int, L: int, itemsize: int) -> Optional[tuple[int, int]]:
+        """(sequences, heads) whose keys and values over L tokens are expanded
+        at a time: as many whole sequences as EXPAND_BYTES hold, else a part of
+        one sequence's heads (a multiple of 8 where it can be: a head's
+        workgroups then stay on one XCD).  None if one head's do not fit."""
+        H = self.n_heads
+        fit = self.EXPAND_BYTES // (2 * L * 128 * itemsize)
+        if fit >= H:
+            return min(B, fit // H), H
+        if fit > 8:
+            fit -= fit % 8
+        return (1, fit) if fit > 0 else None
+
     def _expanded_attention(self, q: torch.Tensor, cache: LatentCache, cos: torch.Tensor, sin: torch.Tensor,
-                            B: int, T: int, start: int, rope_abs: bool) -> torch.Tensor:
+                            B: int, T: int, start: int, rope_abs: bool) -> Optional[torch.Tensor]:
         """Attention output [B * T, H, Dv] of a prompt (q [B * T, H, 192] from
         position ``start``, its own tokens already in the cache): cached
         latents expanded into each head's keys and values once, then causal
-        attention over them (mla.py:427-487)."""
-        H, L = self.n_heads, start + T
-        w_uk, w_uv = self._w_expand()
+        attention over them (mla.py:427-487).  fp32 modules expand by wkv_b's
+        product, ATen's GEMM like their other projections.  None where the
+        keys and values of one head exceed EXPAND_BYTES or the device has no
+        room for them: the latent space needs neither."""
+        H, L, f32 = self.n_heads, start + T, q.dtype == torch.float32
+        groups = self._expand_groups(B, L, q.element_size())
+        if groups is None:
+            return None
+        nb, nh = groups
+        if q.data_ptr() % 16 != 0 or any([st * q.element_size() % 16 != 0 for st in q.stride()[:2]]):
+            q = q.clone(memory_format=torch.contiguous_format)
+        if f32:
+            w = self._padded("wkv_b.rank", self.wkv_b.weight,
+                             lambda: kernels.pad_rank(self.wkv_b.weight.detach(), self.kv_lora_rank))
+        else:
+            w_uk, w_uv = self._w_expand()
         o = torch.empty(B * T, H, self.v_head_dim, dtype=q.dtype, device=q.device)
-        per_seq = 2 * H * L * 128 * q.element_size()
-        step = min(B, max(1, self.EXPAND_BYTES // per_seq))
-        kv = torch.empty(2, step, H, L, 128, dtype=q.dtype, device=q.device)
-        for b0 in range(0, B, step):
-            b1 = min(B, b0 + step)
-            part = LatentCache(cache.ckv[b0:b1], cache.kpe[b0:b1],
-                               None if cache.scale is None else cache.scale[b0:b1], cache.rank)
-            k, v = kv[0, : b1 - b0], kv[1, : b1 - b0]
-            rows = part.ckv[:, None, :L]
-            scale = None if part.scale is None else part.scale[:, :L]
-            kernels.head_product(rows, w_uk, out=k, scale=scale)
-            kernels.head_product(rows, w_uv, out=v, scale=scale)
-            kernels.prompt_attention(q[b0 * T: b1 * T], cos, sin, k, v, part, self.softmax_scale, start=start,
-                                     tokens_per_seq=T, rope_abs=rope_abs, out=o[b0 * T: b1 * T])
-        return o
-
-    def _expanded_attention_f32(self, q: torch.Tensor, cache: LatentCache, cos: torch.Tensor, sin: torch.Tensor,
-                                B: int, T: int, start: int, rope_abs: bool) -> torch.Tensor:
-        """_expanded_attention for an fp32 module: keys and values as wkv_b's
-        product with the cached latents (mla.py:427-437), ATen's GEMM like the
-        module's other fp32 projections."""
-        H, L = self.n_heads, start + T
-        w = self._padded("wkv_b.rank", self.wkv_b.weight,
-                         lambda: kernels.pad_rank(self.wkv_b.weight.detach(), self.kv_lora_rank))
-        o = torch.empty(B * T, H, self.v_head_dim, dtype=q.dtype, device=q.device)
-        per_seq = 2 * H * L * 128 * q.element_size()
-        step = min(B, max(1, self.EXPAND_BYTES // per_seq))
-        for b0 in range(0, B, step):
-            b1 = min(B, b0 + step)
-            part = LatentCache(cache.ckv[b0:b1], cache.kpe[b0:b1], None, cache.rank)
-            kv = torch.nn.functional.linear(part.ckv[:, :L], w).view(b1 - b0, L, H, 256)
-            kernels.prompt_attention_f32(q[b0 * T: b1 * T], cos, sin, kv, part, self.softmax_scale, start=start,
-                                         tokens_per_seq=T, rope_abs=rope_abs, out=o[b0 * T: b1 * T])
+        kw = dict(start=start, tokens_per_seq=T, rope_abs=rope_abs)
+        try:
+            kv = None if f32 else torch.empty(2, nb, nh, L, 128, dtype=q.dtype, device=q.device)
+            for b0 in range(0, B, nb):
+                b1 = min(B, b0 + nb)
+                part = LatentCache(cache.ckv[b0:b1], cache.kpe[b0:b1],
+                                   None if cache.scale is None else cache.scale[b0:b1], cache.rank)
+                for h0 in range(0, H, nh):
+                    h1 = min(H, h0 + nh)
+                    qs, os = q[b0 * T: b1 * T, h0:h1], o[b0 * T: b1 * T, h0:h1]
+                    if f32:
+                        y = torch.nn.functional.linear(part.ckv[:, :L], w[256 * h0: 256 * h1])
+                        kernels.prompt_attention_f32(qs, cos, sin, y.view(b1 - b0, L, h1 - h0, 256), part,
+                                                     self.softmax_scale, out=os, **kw)
+                        del y
+                        continue
+                    k, v = kv[0, : b1 - b0, : h1 - h0], kv[1, : b1 - b0, : h1 - h0]
+                    rows = part.ckv[:, None, :L]
+                    scale = None if part.scale is None else part.scale[:, :L]
+                    kernels.head_product(rows, w_uk[h0:h1], out=k, scale=scale)
+                    kernels.head_product(rows, w_uv[h0:h1], out=v, scale=scale)
+                    kernels.prompt_attention(qs, cos, sin, k, v, part, self.softmax_scale, out=os, **kw)
+        except torch.OutOfMemoryError:
+            return None
         return o
 
     def _forward_kernels(self, x: torch.Tensor, start_pos) -> torch.Tensor:
@@ -995,13 +1011,12 @@ class MLA(nn.Module):
         if (not fused and T > 1 and kernels.expanded_ok(self.rank_pad, Dn, Dv)
                 and not (self.inference_mode and isinstance(start_pos, torch.Tensor))):
             start = int(start_pos) if self.inference_mode else 0
-            o = None
             if x.dtype == torch.bfloat16:
-                if kernels.use_expanded(B, T, start, H, R, self.fp8_cache, self._cus(dev)):
-                    o = self._expanded_attention(q, cache, cos, sin, B, T, start, rope_abs)
-            elif (x.dtype == torch.float32 and not self.fp8_cache
-                  and kernels.use_expanded_f32(B, T, start, H, R, self._cus(dev))):
-                o = self._expanded_attention_f32(q, cache, cos, sin, B, T, start, rope_abs)
+                use = kernels.use_expanded(B, T, start, H, R, self.fp8_cache, self._cus(dev))
+            else:
+                use = (x.dtype == torch.float32 and not self.fp8_cache
+                       and kernels.use_expanded_f32(B, T, start, H, R, self._cus(dev)))
+            o = self._expanded_attention(q, cache, cos, sin, B, T, start, rope_abs) if use else None
             if o is not None:
                 return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
 

@@ -284,3 +284,105 @@ def test_later_nonfinite_tokens_stay_out(gpu, dtype, where, T, start, bad):
     got = out.double().view(B, T, H, 128).transpose(1, 2)
     assert not bool(torch.isfinite(got[hit]).any())
     assert bool(((got - ref).abs() <= bound)[~hit].all()), float(((got - ref).abs() - bound)[~hit].max())
+
+
+@pytest.mark.parametrize("dtype,cache,H", [(torch.bfloat16, None, 12), (torch.bfloat16, "fp8_e4m3", 16),
+                                           (torch.float32, None, 12)])
+@pytest.mark.parametrize("heads_at_once", [11, 8, 5, 1])
+def test_expansion_in_head_groups(gpu, dtype, cache, H, heads_at_once, monkeypatch):
+    """With less room than one sequence's keys and values need, heads go in
+    groups that fit it: bf16 output bits as in one piece (fp32: another GEMM
+    shape, 1e-5 of the scale)."""
+    say(f"head groups {dtype} cache={cache} H={H} at once={heads_at_once}")
+    B, T, start = 2, 300, 200
+    m = MLA(MLAConfig(n_embd=512, n_head=H, max_batch_size=B, max_seq_len=512), cache_dtype=cache)
+    g = torch.Generator().manual_seed(H)
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            if name.endswith("weight") and "norm" not in name:
+                p.copy_(torch.randn(p.shape, generator=g) * 0.03)
+    m.eval().to(dtype).to(gpu)
+    m.set_inference_mode(True)
+    per_head = 2 * (start + T) * 128 * (2 if dtype == torch.bfloat16 else 4)
+    name = "prompt_attention" if dtype == torch.bfloat16 else "prompt_attention_f32"
+    calls, real = [], getattr(kernels, name)
+
+    def spy(q, cos, sin, *kv_cache, **k):
+        room = sum(t.numel() * t.element_size() for t in kv_cache if isinstance(t, torch.Tensor))
+        assert room <= m.EXPAND_BYTES
+        calls.append(q.shape[1])
+        return real(q, cos, sin, *kv_cache, **k)
+
+    monkeypatch.setattr(kernels, name, spy)
+    monkeypatch.setattr(kernels, "use_expanded", lambda *a, **k: True)
+    monkeypatch.setattr(kernels, "use_expanded_f32", lambda *a, **k: True)
+    x0, x = (torch.randn(B, t, 512, generator=g).to(dtype).to(gpu) for t in (start, T))
+    outs = []
+    for room in (B * H * per_head, heads_at_once * per_head + per_head // 2):
+        m.EXPAND_BYTES = room
+        calls.clear()
+        with torch.no_grad():
+            m.prefill_cache(x0, 0)
+            outs.append(m(x, start))
+        torch.cuda.synchronize()
+        if len(outs) == 1:
+            assert calls == [H]
+    step = 8 if 8 < heads_at_once < 16 else heads_at_once
+    assert calls == B * [min(step, H - h) for h in range(0, H, step)], calls
+    if dtype == torch.bfloat16:
+        assert torch.equal(*outs)
+    else:
+        assert float((outs[0] - outs[1]).abs().max()) <= 1e-5 * float(outs[0].abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_no_room_for_the_expansion(gpu, dtype, monkeypatch):
+    """No room for one head's keys and values, by EXPAND_BYTES or on the
+    device: the call is the latent route's, bit for bit."""
+    m = MLA(MLAConfig(n_embd=512, max_batch_size=1, max_seq_len=400))
+    g = torch.Generator().manual_seed(9)
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            if name.endswith("weight") and "norm" not in name:
+                p.copy_(torch.randn(p.shape, generator=g) * 0.03)
+    m.eval().to(dtype).to(gpu)
+    m.set_inference_mode(True)
+    x = torch.randn(1, 400, 512, generator=g).to(dtype).to(gpu)
+    rule = "use_expanded" if dtype == torch.bfloat16 else "use_expanded_f32"
+    with torch.no_grad():
+        monkeypatch.setattr(kernels, rule, lambda *a, **k: False)
+        want = m(x, 0)
+        monkeypatch.setattr(kernels, rule, lambda *a, **k: True)
+        expanded = m(x, 0)
+        m.EXPAND_BYTES = 1000
+        assert torch.equal(m(x, 0), want)
+        m.EXPAND_BYTES = MLA.EXPAND_BYTES
+        assert torch.equal(m(x, 0), expanded)
+
+        def full(*a, **k):
+            raise torch.OutOfMemoryError("planted")
+
+        monkeypatch.setattr(kernels, "head_product" if dtype == torch.bfloat16 else "prompt_attention_f32",
+                            lambda x, *a, real=kernels.head_product, **k: real(x, *a, **k) if x.dim() == 3 and
+                            dtype == torch.bfloat16 else full())
+        assert torch.equal(m(x, 0), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_query_rows_of_any_alignment(gpu, dtype):
+    """A query projection put in wq's place may return a view at any address."""
+
+    class Offset(torch.nn.Linear):
+        def forward(self, x):
+            y = super().forward(x)
+            out = torch.zeros(*y.shape[:-1], y.shape[-1] + 3, dtype=y.dtype, device=y.device)
+            out[..., 3:] = y
+            return out[..., 3:]
+
+    m = MLA(MLAConfig(n_embd=512, kv_lora_rank=640, max_batch_size=1, max_seq_len=512)).eval().to(dtype).to(gpu)
+    m.set_inference_mode(True)
+    x = torch.randn(1, 512, 512, device=gpu).to(dtype)
+    with torch.no_grad():
+        want = m(x, 0)
+        m.wq.__class__ = Offset
+        assert torch.equal(m(x, 0), want)

@@ -90,3 +90,24 @@ def test_min_chunk_by_dtype_rank_and_length():
     m = MLA(MLAConfig(kv_lora_rank=640, max_batch_size=1, max_seq_len=64)).to(torch.bfloat16)
     m._num_cus = 256
     assert m._split_plan(1, 2000, torch.device("cpu")) == (32, 64)
+
+
+def test_expansion_groups():
+    """Keys and values of a prompt never take more than EXPAND_BYTES: whole
+    sequences while they fit, then a sequence's heads in groups (multiples of
+    8 where it can be), and none where one head's exceed it."""
+    for heads, itemsize in ((16, 2), (32, 2), (12, 4), (5, 2)):
+        m = MLA(MLAConfig(n_head=heads, max_batch_size=1, max_seq_len=8))
+        for B, L in ((1, 1), (4, 4096), (64, 512), (1, 131072), (3, 200000), (1, 1 << 20), (1, 3 << 20)):
+            head = 2 * L * 128 * itemsize
+            got = m._expand_groups(B, L, itemsize)
+            if head > m.EXPAND_BYTES:
+                assert got is None
+                continue
+            nb, nh = got
+            assert nb * nh * head <= m.EXPAND_BYTES and 1 <= nb <= B and 1 <= nh <= heads
+            assert nh == heads or (nb == 1 and (nh <= 8 or nh % 8 == 0))
+            room = m.EXPAND_BYTES // head
+            assert nh > room - 8 if nh < heads else nb == min(B, room // heads)
+    m = MLA(MLAConfig(n_head=32, max_batch_size=1, max_seq_len=8))
+    assert m._expand_groups(1, 132096, 2) == (1, 7)  # 2.1 GB in one piece
