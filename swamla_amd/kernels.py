@@ -761,18 +761,17 @@ def use_expanded_f32(n_seq: int, tokens_per_seq: int, start: int, heads: int, ra
                      num_cus: int = 256) -> bool:
     """use_expanded for an fp32 module, whose latent path is the per-row VALU
     kernel and batched products: only a few tokens behind a long prefix stay
-    there.  Microseconds on 256 CUs, 16 heads, rank 256; whole forwards
-    expanded / latent: 1 x 512 from 0 128 / 608, 1 x 2 46 / 74, 2 x 1024 402 /
-    3070, 1 x 256 at 2000 231 / 2252, 1 x 16 at 4000 299 / 321.  The expansion
-    is a GEMM at about 47 TFLOP/s, a workgroup of the attention takes 5 us per
-    eight tiles; the VALU kernel 3.5 ms per million pairs, and 0.8 us per token
-    of its longest split.  Head counts other than 16 come over past 320
-    tokens (1 x 512 at 12 heads 118 / 606); up to there they stay on the
-    16-head launches over padded heads that the tests of those modules count
-    (2 x 160 tokens)."""
+    there.  Microseconds on 256 CUs.  The expansion is a GEMM at about 47
+    TFLOP/s, a workgroup of the attention takes 5 us per eight tiles; the VALU
+    kernel 3.5 ms per million pairs and 16 heads, and 0.8 us per token of its
+    longest split.  Whole forwards, graph-replayed, expanded / latent, 16 heads
+    at rank 256: 1 x 2 from 0 45 / 73, 1 x 512 128 / 608, 2 x 1024 402 / 3070,
+    1 x 16 at 4000 291 / 315, 1 x 8 at 4000 290 / 196; at 5 / 12 / 32 heads, 2 x
+    160 from 0 68 / 233, 83 / 252, 128 / 456, and 1 x 8 at 4000 251 / 174, 274 /
+    200, 358 / 312.  Over 5 to 40 heads and ranks 64, 256 and 640 it took the
+    faster route but where they are within 18 % of each other (it then stays
+    in the latent space)."""
     B, T, L = n_seq, tokens_per_seq, start + tokens_per_seq
-    if heads != H and B * T <= 320:
-        return False
     rp = padded_rank(rank)
     pairs = B * (T * start + T * (T + 1) / 2) * 1e-6
     expand = 10 + 2.0 * B * L * heads * 256 * rp / 47e6

@@ -380,6 +380,9 @@ def test_module_other_head_counts(gpu, dtype, n_head, dim, nope, rank, monkeypat
         return real_mp(o_lat, *a, **k)
 
     monkeypatch.setattr(kernels, "merge_project", spy_mp)
+    # the launches of the latent route are counted below, which an fp32 prompt of
+    # this size does not take by itself (test_module_fp32_prompt_head_counts)
+    monkeypatch.setattr(kernels, "use_expanded_f32", lambda *a, **k: False)
     g = torch.Generator().manual_seed(42 + n_head)
     x = torch.randn(2, 160, dim, generator=g).to(dtype)
     xs = [x.to(gpu)]
@@ -401,6 +404,25 @@ def test_module_other_head_counts(gpu, dtype, n_head, dim, nope, rank, monkeypat
         assert fused == [max(n_head, 16)] * 6, fused
     else:
         assert fused == [], fused
+
+
+@pytest.mark.parametrize("n_head", [5, 12, 16, 32])
+@pytest.mark.parametrize("T", [2, 64, 160])
+def test_module_fp32_prompt_head_counts(gpu, n_head, T, monkeypatch):
+    """Short fp32 prompts of any head count run over expanded keys and values
+    and match the reference; cache rows bit-exact."""
+    say(f"fp32 prompt n_head={n_head} T={T}")
+    cfg = MLAConfig(n_embd=512, n_head=n_head, max_batch_size=2, max_seq_len=192)
+    ref, ours = make_pair(cfg, 51 + n_head, torch.float32, gpu, ln_random=True)
+    calls = []
+    real = kernels.prompt_attention_f32
+    monkeypatch.setattr(kernels, "prompt_attention_f32", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    x = torch.randn(2, T, 512, generator=torch.Generator().manual_seed(T))
+    with torch.no_grad():
+        close(ours(x.to(gpu), 0), ref(x, 0), torch.float32)
+    torch.cuda.synchronize()
+    assert len(calls) == 1
+    assert_cache_bits(ours, [x.to(gpu)], torch.float32)
 
 
 def test_out_of_range_positions_raise(gpu):

@@ -111,3 +111,28 @@ def test_expansion_groups():
             assert nh > room - 8 if nh < heads else nb == min(B, room // heads)
     m = MLA(MLAConfig(n_head=32, max_batch_size=1, max_seq_len=8))
     assert m._expand_groups(1, 132096, 2) == (1, 7)  # 2.1 GB in one piece
+
+
+def test_fp32_route_of_prompts():
+    """use_expanded_f32 against measured forwards (us expanded / latent): short
+    prompts of every head count expand, a few tokens behind a long prefix do
+    not, and nothing hangs on one head count or one size."""
+    f = kernels.use_expanded_f32
+    for heads in (5, 8, 12, 16, 32, 40):
+        for rank in (64, 256, 640):
+            for B, T in ((1, 2), (1, 64), (2, 160), (1, 320), (1, 321)):
+                assert f(B, T, 0, heads, rank), (heads, rank, B, T)
+            assert f(1, 64, 2000, heads, rank)  # 176-397 / 168-2834
+            assert not f(1, 2, 4000, heads, rank)  # 233-631 / 73-350
+    assert f(1, 16, 4000, 12, 256) and not f(1, 8, 4000, 12, 256)  # 275 / 308, 274 / 200
+
+
+def test_bf16_route_of_prompts():
+    """use_expanded on both sides of its crossings, where whole forwards were
+    timed on each route (its docstring)."""
+    f = kernels.use_expanded
+    yes = [(1, 640, 0, 16, 256), (4, 4096, 0, 16, 256), (2, 512, 8192, 16, 256), (8, 1001, 0, 16, 444),
+           (4, 2048, 0, 32, 256, True)]
+    no = [(1, 256, 0, 16, 256), (1, 512, 0, 16, 256), (32, 64, 1024, 16, 256), (32, 64, 4032, 16, 256), (1, 256, 4096, 16, 256)]
+    assert [f(*a) for a in yes] == [True] * len(yes)
+    assert [f(*a) for a in no] == [False] * len(no)
