@@ -62,7 +62,11 @@ enum {
 enum { SWAMLA_DTYPE_F32 = 0, SWAMLA_DTYPE_BF16 = 1, SWAMLA_DTYPE_FP8 = 2 };
 
 /* ABI revision of the loaded library; callers compare it with
- * SWAMLA_ABI_VERSION.  No reference counterpart (the reference has no FFI). */
+ * SWAMLA_ABI_VERSION.  It changes when an entry point here changes; entry
+ * points added since (the last ones: mla_merge_project_wide,
+ * mla_head_product_rows, mla_prompt_attn, mla_prompt_attn_f32) leave it, so a
+ * caller that needs one looks its name up.  No reference counterpart (the
+ * reference has no FFI). */
 int mla_abi_version(void);
 
 /* Message describing the last non-zero return on this thread ("" if none).

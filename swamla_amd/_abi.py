@@ -172,10 +172,13 @@ def lib() -> ctypes.CDLL:
                 "(there is no CPU or eager fallback for this path)"
             )
         handle = ctypes.CDLL(LIB_PATH)
-        _declare(handle)
-        got = handle.mla_abi_version()
+        missing = [name for name in EXPORTED_SYMBOLS if not hasattr(handle, name)]
+        got = None if "mla_abi_version" in missing else handle.mla_abi_version()
         if got != ABI_VERSION:
             raise RuntimeError(f"{LIB_NAME} ABI version {got} != expected {ABI_VERSION}")
+        if missing:  # entry points are added without a new revision
+            raise RuntimeError(f"{LIB_PATH} is older than this package (it lacks {', '.join(missing)}): build it again")
+        _declare(handle)
         _lib = handle
     return _lib
 

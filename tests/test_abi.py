@@ -5,6 +5,7 @@ import ctypes
 import glob
 import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -37,6 +38,23 @@ def test_exports_every_declared_symbol(lib):
 
 def test_abi_version(lib):
     assert lib.mla_abi_version() == _abi.ABI_VERSION == 6
+
+
+@pytest.mark.parametrize("source,message", [
+    ("int mla_abi_version(void) { return 6; } int mla_append(void) { return 0; }", "older than this package.*mla_prompt_attn"),
+    ("int mla_abi_version(void) { return 5; }", "ABI version 5"),
+    ("int something_else(void) { return 0; }", "ABI version None"),
+])
+def test_other_libraries_are_named(tmp_path, monkeypatch, source, message):
+    """A library of another revision, or of this one without the entry points
+    added since, is refused with the reason."""
+    c, so = tmp_path / "lib.c", tmp_path / "lib.so"
+    c.write_text(source)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(c), "-o", str(so)], check=True)
+    monkeypatch.setattr(_abi, "LIB_PATH", str(so))
+    monkeypatch.setattr(_abi, "_lib", None)
+    with pytest.raises(RuntimeError, match=message):
+        _abi.lib()
 
 
 def _append(lib, **kw):
