@@ -92,16 +92,18 @@ __global__ __launch_bounds__(256, (HpGeo<NB, FP8 ? 1 : 2>::kPerCu)) void mla_hea
   const int stride = gridDim.x;
 
   // columns: with x shared by the heads the units of 32 columns run over
-  // (head, n) in one sequence; else a group stays within one head
+  // (head, n) in one sequence; else a group stays within one head (groups past
+  // the last head of the grid's last row: no columns)
+  const int grp = blockIdx.y + gridDim.y * blockIdx.z;
   int h, n0;
   if (a.shared) {
-    const int u = (static_cast<int>(blockIdx.y) * 4 + w) * 32;
+    const int u = (grp * 4 + w) * 32;
     h = u / a.N;
     n0 = u - h * a.N;
   } else {
     const int gph = (a.N + 127) / 128;
-    h = blockIdx.y / gph;
-    n0 = ((blockIdx.y - h * gph) * 4 + w) * 32;
+    h = grp / gph;
+    n0 = ((grp - h * gph) * 4 + w) * 32;
   }
   const bool cols = h < a.H && n0 < a.N;  // uniform; a wave without columns still copies its part of the tiles
   h = min(h, a.H - 1);
@@ -247,10 +249,11 @@ int launch_instance(const HeadProductArgs& a, int n_cus, hipStream_t s) {
   const int64_t n_tiles = static_cast<int64_t>((a.M + G::kRows - 1) / G::kRows) * a.B;
   const int64_t groups = a.shared ? (static_cast<int64_t>(a.H) * a.N + 127) / 128
                                   : static_cast<int64_t>(a.H) * ((a.N + 127) / 128);
-  if (n_tiles > (int64_t(1) << 30) || groups > 65535) return -1;
+  if (n_tiles > (int64_t(1) << 30) || groups > (int64_t(1) << 30)) return -1;
+  const int64_t gy = groups > 32768 ? 32768 : groups, gz = (groups + gy - 1) / gy;
   int64_t gx = (static_cast<int64_t>(n_cus) * G::kPerCu + groups - 1) / groups;
   gx = gx < 1 ? 1 : (gx > n_tiles ? n_tiles : gx);
-  hipLaunchKernelGGL((mla_head_product_kernel<NB, FP8>), dim3(static_cast<uint32_t>(gx), static_cast<uint32_t>(groups)),
+  hipLaunchKernelGGL((mla_head_product_kernel<NB, FP8>), dim3(static_cast<uint32_t>(gx), static_cast<uint32_t>(gy), static_cast<uint32_t>(gz)),
                      dim3(256), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
@@ -267,7 +270,7 @@ int launch_head_product(const HeadProductArgs& a0, int n_cus, hipStream_t s) {
   HeadProductArgs a = a0;
   // 16-byte stores where every lane's run of columns starts on 16 bytes
   a.y_wide = reinterpret_cast<uintptr_t>(a.y) % 16 == 0 && (a.y_rs | a.y_hs | a.y_bs | a.N) % 8 == 0;
-  a.shared = a.x_hs == 0 && a.N % 64 == 0;
+  a.shared = a.x_hs == 0 && a.N % 64 == 0 && static_cast<int64_t>(a.H) * a.N <= (int64_t(1) << 30);
   if (a.K % 64 != 0 || (a.x_scale && !a.shared)) return -1;
   switch (a.K / 64) {
     case 1: return launch_nb<1>(a, n_cus, s);

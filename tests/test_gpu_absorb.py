@@ -104,6 +104,25 @@ def test_head_counts(gpu, H):
     check(out, ref_head_product(x, w))
 
 
+@pytest.mark.parametrize("N", [16384, 16388])
+@pytest.mark.parametrize("shared", [False, True])
+def test_more_column_groups_than_a_grid_row(gpu, N, shared):
+    """600 heads of 16,384 columns: 76,800 groups of 128 columns, past the
+    65,535 of one grid dimension (every head with the same weight rows; with
+    ``shared`` also the same x row)."""
+    say(f"head_product 600 heads x {N} columns, shared={shared}")
+    g = torch.Generator(device=gpu).manual_seed(N)
+    x = torch.randn(2, 1 if shared else 600, 64, generator=g, device=gpu).to(torch.bfloat16).expand(2, 600, 64)
+    w = (torch.randn(1, N, 64, generator=g, device=gpu) * 0.06).to(torch.bfloat16)
+    out = torch.full((2, 600, N), 7.0, dtype=torch.bfloat16, device=gpu)
+    kernels.head_product(x, w.expand(600, N, 64), out=out)
+    torch.cuda.synchronize()
+    for m in range(2):
+        ref = x[m].double() @ w[0].double().T
+        bar = 2.0 ** -7 * ref.abs() + 64 * 2.0 ** -24 * (x[m].double().abs() @ w[0].double().abs().T)
+        assert bool(((out[m].double() - ref).abs() <= bar).all())
+
+
 def test_strided_output_leaves_gaps_untouched(gpu):
     """y rows wider than H * N: the columns between heads are not written."""
     M, H, K, N = 200, 4, 128, 64
