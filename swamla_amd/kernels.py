@@ -769,8 +769,8 @@ def use_expanded_f32(n_seq: int, tokens_per_seq: int, start: int, heads: int, ra
     1 x 16 at 4000 291 / 315, 1 x 8 at 4000 290 / 196; at 5 / 12 / 32 heads, 2 x
     160 from 0 68 / 233, 83 / 252, 128 / 456, and 1 x 8 at 4000 251 / 174, 274 /
     200, 358 / 312.  Over 5 to 40 heads and ranks 64, 256 and 640 it took the
-    faster route but where they are within 18 % of each other (it then stays
-    in the latent space)."""
+    faster route but where the two are within a fifth of each other (it then
+    stays in the latent space)."""
     B, T, L = n_seq, tokens_per_seq, start + tokens_per_seq
     rp = padded_rank(rank)
     pairs = B * (T * start + T * (T + 1) / 2) * 1e-6

@@ -48,3 +48,22 @@ def check_lse(lse, ref, atol=LSE_ATOL):
     err = torch.where(both_inf, torch.zeros_like(lse), (lse - ref).abs())
     assert not bool(torch.isnan(err).any()), "NaN log-sum-exp"
     assert float(err.max()) <= atol, f"log-sum-exp off by {float(err.max()):.3e} (> {atol})"
+
+
+def wide_bars(s, p, lat, ref, score_terms):
+    """Bounds for the channel-split bf16 attention of one row against fp64
+    (s, p [H, L] scores and weights, lat [L, R], ref = p @ lat): per element,
+    and per head the RMS over its channels.
+
+    A weight is rounded to bf16 (2^-9), for e4m3 once more after the token's
+    scale, and normalised by the rounded weights' sum: each within 3 x 2^-9.
+    ``score_terms`` [H, L] is the sum of |products| of a score: fp32 sums of
+    R + 64 of them are within (R + 64) 2^-24 of it.  The output is rounded
+    once (2^-9 of it).  The errors of different tokens are independent, so
+    over the channels they add up as squares: sqrt(sum p^2 lat^2), which falls
+    with the length as one lost step's share of the output does not."""
+    e = torch.expm1(2 * (lat.shape[1] + 64) * 2.0 ** -24 * score_terms.amax(-1, keepdim=True))
+    w = 3 * 2.0 ** -9 + e
+    lim = (p @ lat.abs()) * w + 2.0 ** -8 * ref.abs()
+    rms = lambda t: t.square().mean(-1, keepdim=True).sqrt()
+    return lim, w * (rms((p.square() @ lat.square()).sqrt()) + rms(ref))

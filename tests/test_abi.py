@@ -343,6 +343,148 @@ def test_merge_project_rejects(lib, kw, code):
     assert lib.mla_last_error().decode()
 
 
+@pytest.mark.parametrize(
+    "kw,code",
+    [
+        (dict(R=512, o_hs=1024), -2),  # up to 512: mla_merge_project
+        (dict(R=1025), -2),
+        (dict(dt=0), -2),
+        (dict(Dv=64), -2),
+        (dict(ns=0), -1),
+        (dict(n_rows=-1), -1),
+        (dict(o_part=None), -1),
+        (dict(row_seq=None), -1),
+        (dict(o_lat=None), -1),
+        (dict(cs=0), -1),
+        (dict(o_hs=640), -1),  # below R_pad = 704
+        (dict(w_rs=640), -1),
+        (dict(y_hs=64), -1),
+        (dict(w=FAKE + 8), -3),
+        (dict(o_rs=4100), -3),
+        (dict(plan=FAKE + 2), -3),
+    ],
+)
+def test_merge_project_wide_rejects(lib, kw, code):
+    args = dict(o_part=FAKE, lse=FAKE, o_lat=FAKE, o_rs=16 * 704, o_hs=704, kv_len=FAKE, row_seq=FAKE, sp=None, T=1,
+                cb=4, cs=64, n_rows=8, H=16, R=650, ns=4, mc=64, plan=None, w=FAKE, w_rs=704, w_hs=90112, Dv=128,
+                y=FAKE, y_rs=2048, y_hs=128, dt=1, stream=None)
+    args.update(kw)
+    assert lib.mla_merge_project_wide(*args.values()) == code
+    assert "mla_merge_project_wide" in lib.mla_last_error().decode() or kw == dict(R=1025)
+    args.update(n_rows=0, R=650, Dv=128, dt=1, ns=4)
+    assert lib.mla_merge_project_wide(*args.values()) == 0
+
+
+def _head_product_rows(lib, **kw):
+    args = dict(x=FAKE, x_rs=256, x_bs=16384, sc=None, s_bs=0, w=FAKE, w_rs=256, w_hs=32768, y=FAKE, y_rs=128,
+                y_hs=8192, y_bs=131072, B=2, M=64, N=128, K=256, H=16, dt=1, stream=None)
+    args.update(kw)
+    return lib.mla_head_product_rows(*args.values())
+
+
+@pytest.mark.parametrize(
+    "kw,code",
+    [
+        (dict(dt=0), -2),
+        (dict(K=0), -2),
+        (dict(K=1088, x_rs=1088, w_rs=1088), -2),
+        (dict(K=96), -2),
+        (dict(N=96), -2),
+        (dict(B=-1), -1),
+        (dict(M=-1), -1),
+        (dict(H=32769), -1),  # H N > 2^22
+        (dict(x=None), -1),
+        (dict(w=None), -1),
+        (dict(y=None), -1),
+        (dict(dt=2), -1),  # e4m3 rows without scales
+        (dict(sc=FAKE), -1),  # scales without e4m3 rows
+        (dict(x_rs=128), -1),
+        (dict(w_rs=128), -1),
+        (dict(x_bs=-256), -1),
+        (dict(y_rs=-4), -1),
+        (dict(x=FAKE + 8), -3),
+        (dict(w=FAKE + 8), -3),
+        (dict(y=FAKE + 4), -3),
+        (dict(x_rs=260), -3),
+        (dict(dt=2, sc=FAKE, x_rs=264), -3),  # e4m3: strides of 16 codes
+        (dict(dt=2, sc=FAKE + 2), -3),
+        (dict(w_hs=32772), -3),
+        (dict(y_hs=8194), -3),
+    ],
+)
+def test_head_product_rows_rejects(lib, kw, code):
+    assert _head_product_rows(lib, **kw) == code
+    assert "mla_head_product_rows" in lib.mla_last_error().decode()
+
+
+def test_head_product_rows_empty_is_a_noop(lib):
+    for kw in (dict(B=0), dict(M=0), dict(N=0), dict(H=0)):
+        assert _head_product_rows(lib, x=None, w=None, y=None, **kw) == 0
+
+
+def _prompt(lib, f32, **kw):
+    args = dict(q=FAKE, q_rs=3072, q_hs=192, cos=FAKE, sin=FAKE, rope_len=64, k=FAKE, v=FAKE, kpe=FAKE, cb=2, cs=64,
+                B=2, T=32, start=16, rope_abs=0, H=16, Dn=128, P=64, Dv=128, sm=0.07, o=FAKE, o_rs=2048, o_hs=128,
+                dt=1, stream=None)
+    args.update(kw)
+    if f32:
+        kv = args.pop("v")
+        args["k"] = None if kv is None else args["k"]
+        del args["dt"]
+        return lib.mla_prompt_attn_f32(*args.values())
+    return lib.mla_prompt_attn(*args.values())
+
+
+@pytest.mark.parametrize("f32", [False, True], ids=["bf16", "fp32"])
+@pytest.mark.parametrize(
+    "kw,code",
+    [
+        (dict(Dn=64), -2),
+        (dict(P=32), -2),
+        (dict(Dv=64), -2),
+        (dict(B=-1), -1),
+        (dict(T=-1), -1),
+        (dict(H=-1), -1),
+        (dict(start=-1), -1),
+        (dict(q=None), -1),
+        (dict(k=None), -1),
+        (dict(v=None), -1),
+        (dict(kpe=None), -1),
+        (dict(sin=None), -1),
+        (dict(o=None), -1),
+        (dict(cb=1), -1),  # two sequences in a cache of one
+        (dict(start=33), -1),  # 33 + 32 tokens in a cache of 64
+        (dict(start=2**31 - 1), -1),
+        (dict(cs=2**31), -1),
+        (dict(rope_len=0), -1),
+        (dict(sm=0.0), -1),
+        (dict(sm=float("nan")), -1),
+        (dict(q_hs=128), -1),
+        (dict(o_hs=64), -1),
+        (dict(q_rs=-3072), -1),
+        (dict(q=FAKE + 8), -3),
+        (dict(k=FAKE + 8), -3),
+        (dict(kpe=FAKE + 8), -3),
+        (dict(o=FAKE + 8), -3),
+        (dict(cos=FAKE + 4), -3),
+        (dict(q_rs=3074), -3),
+        (dict(o_rs=2050), -3),
+    ],
+)
+def test_prompt_attn_rejects(lib, f32, kw, code):
+    assert _prompt(lib, f32, **kw) == code
+    name = "mla_prompt_attn_f32:" if f32 else "mla_prompt_attn:"
+    assert lib.mla_last_error().decode().startswith(name)
+
+
+def test_prompt_attn_other_dtypes_and_empty(lib):
+    assert _prompt(lib, False, dt=0) == -2 and _prompt(lib, False, dt=2) == -2
+    assert _prompt(lib, False, q_rs=3076) == -3  # bf16: multiples of 8; fp32: of 4
+    for f32 in (False, True):
+        for kw in (dict(B=0), dict(T=0), dict(H=0)):
+            assert _prompt(lib, f32, q=None, k=None, v=None, o=None, **kw) == 0
+
+
 def test_merge_project_single_split_needs_no_partials(lib):
     # validation passes without partial buffers when n_splits == 1 (n_rows = 0: no launch)
     assert _merge_project(lib, ns=1, o_part=None, lse=None, n_rows=0) == 0

@@ -70,6 +70,9 @@ SCRATCH_BUDGET = {
     "mla_merge_project_kernel": 0,
     "mla_merge_kernel": 0,
     "mla_append_g16_kernel": 0,
+    "mla_prompt_kernel": 0,
+    "mla_prompt_f32_kernel": 0,
+    "mla_head_product_kernel": 0,
     "mla_prefill_m32": 8,  # the persistent item loop re-loads a few values once per query group
 }
 
