@@ -675,6 +675,14 @@ class MLA(nn.Module):
         return self._derived("w_uk_t.wide", self.wkv_b.weight,
                              lambda: torch.cat([w, w.new_zeros((kernels.H - H,) + tuple(w.shape[1:]))], 0))
 
+    def _dropped(self, out: torch.Tensor) -> torch.Tensor:
+        """resid_dropout (mla.py:495).  The call (2 us of host time) is left
+        out only where it is nn.Dropout's own identity."""
+        drop = self._modules.get("resid_dropout")
+        if drop is None or drop.training or not _plain(drop, nn.Dropout):
+            return self.resid_dropout(out)
+        return out
+
     def _check_geometry(self) -> None:
         if (self.n_heads < 1 or self.qk_rope_head_dim != kernels.P
                 or not 1 <= self.kv_lora_rank <= kernels.MAX_RANK):
@@ -785,7 +793,7 @@ class MLA(nn.Module):
             self._advance_folded = adv is not None
         else:
             out = kernels.linear(o, self._wo_fused(), bias=wo_b).view(B, T, self.dim)
-        return self.resid_dropout(out)
+        return self._dropped(out)
 
     @staticmethod
     def _mask_key(mask: torch.Tensor, T: int) -> tuple:
@@ -1018,7 +1026,7 @@ class MLA(nn.Module):
                        and kernels.use_expanded_f32(B, T, start, H, R, self._cus(dev)))
             o = self._expanded_attention(q, cache, cos, sin, B, T, start, rope_abs) if use else None
             if o is not None:
-                return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
+                return self._dropped(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
 
         n_splits, min_chunk, balance = self._decode_plan(
             n, max_len, dev, isinstance(start_pos, torch.Tensor) and self.inference_mode, dtype=x.dtype)
@@ -1112,4 +1120,4 @@ class MLA(nn.Module):
             kernels.head_product(o_lat[:, :H], self._w_uv(), out=o.view(n, H, Dv))
         else:
             o = torch.bmm(o_lat[:, :H].transpose(0, 1), w_uv_t).transpose(0, 1).reshape(n, H * Dv)  # [n, H*Dv]
-        return self.resid_dropout(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495
+        return self._dropped(self.wo(o.view(B, T, H * Dv)))  # mla.py:490-495

@@ -56,6 +56,18 @@ def test_resid_dropout_is_called(gpu, rank, T, dtype):
         finally:
             handle.remove()
         assert m.resid_dropout in seen
+        for register in (m.resid_dropout.register_forward_hook, m.resid_dropout.register_forward_pre_hook):
+            seen.clear()
+            handle = register(lambda mod, *a: seen.append(mod))
+            m(x, 0)
+            handle.remove()
+            assert seen == [m.resid_dropout]
+        m.resid_dropout.forward = lambda x: 0.25 * x
+        assert torch.equal(m(x, 0), 0.25 * want)
+        del m.resid_dropout.forward
+        assert torch.equal(m(x, 0), want)
+        m.resid_dropout = type("Sub", (nn.Dropout,), {"forward": lambda self, x: 2 * x})()
+        assert torch.equal(m.eval()(x, 0), 2 * want)
         m.resid_dropout = Halve()
         got = m(x, 0)
     torch.cuda.synchronize()
