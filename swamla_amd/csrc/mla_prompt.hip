@@ -354,6 +354,10 @@ __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs
     stream(Y{}, N{}, lds_k, 0);
     softmax(0);
   }
+  // Puts the loop's barrier 4 bytes past a multiple of 8 (most instructions
+  // there take 8 bytes): on a multiple of 8 a whole forward took 549 instead of
+  // 556 us at 4 x 4096 tokens, but 234 instead of 228 at 8 x 1001.
+  asm volatile(".p2align 3\n\ts_nop 0" ::: "memory");
   for (int j = 0; j < n_tiles; ++j) {
     st_tile_barrier();  // K tile j + 1 and V tile j complete; K tile j and V tile j - 1 consumed
     if (j + 2 < n_tiles) copy_k(j + 2);
@@ -369,12 +373,12 @@ __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs
   if (w_tiles == 0) return;  // uniform: no query
 
   // Columns whose sums hold a NaN (finite x 0 adds nothing): see prompt_row.
-  float nan_sum = 0.f;
+  float z[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb)
+  for (int r = 0; r < 16; ++r)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) nan_sum = __builtin_fmaf(oacc[cb][r], 0.f, nan_sum);
-  const uint64_t bad2 = __ballot(t_w + n < a.T && nan_sum != 0.f);
+    for (int cb = 0; cb < 4; ++cb) z[cb] = __builtin_fmaf(oacc[cb][r], 0.f, z[cb]);
+  const uint64_t bad2 = __ballot(t_w + n < a.T && (z[0] + z[1]) + (z[2] + z[3]) != 0.f);
   uint32_t bad = static_cast<uint32_t>(bad2) | static_cast<uint32_t>(bad2 >> 32);
 
   // Lane (n, hf) holds positions 32 cb + 8 r4 + 4 hf + e of its query's

@@ -931,7 +931,8 @@ class MLA(nn.Module):
         if groups is None:
             return None
         nb, nh = groups
-        if q.data_ptr() % 16 != 0 or any([st * q.element_size() % 16 != 0 for st in q.stride()[:2]]):
+        whole = nb >= B and nh == H
+        if q.data_ptr() % 16 != 0 or (q.stride(0) | q.stride(1)) * q.element_size() % 16 != 0:
             q = q.clone(memory_format=torch.contiguous_format)
         if f32:
             w = self._padded("wkv_b.rank", self.wkv_b.weight,
@@ -948,18 +949,18 @@ class MLA(nn.Module):
                                    None if cache.scale is None else cache.scale[b0:b1], cache.rank)
                 for h0 in range(0, H, nh):
                     h1 = min(H, h0 + nh)
-                    qs, os = q[b0 * T: b1 * T, h0:h1], o[b0 * T: b1 * T, h0:h1]
+                    qs, os = (q, o) if whole else (q[b0 * T: b1 * T, h0:h1], o[b0 * T: b1 * T, h0:h1])
                     if f32:
-                        y = torch.nn.functional.linear(part.ckv[:, :L], w[256 * h0: 256 * h1])
+                        y = torch.nn.functional.linear(part.ckv[:, :L], w if whole else w[256 * h0: 256 * h1])
                         kernels.prompt_attention_f32(qs, cos, sin, y.view(b1 - b0, L, h1 - h0, 256), part,
                                                      self.softmax_scale, out=os, **kw)
                         del y
                         continue
-                    k, v = kv[0, : b1 - b0, : h1 - h0], kv[1, : b1 - b0, : h1 - h0]
+                    k, v = kv[:, : b1 - b0, : h1 - h0].unbind(0)
                     rows = part.ckv[:, None, :L]
                     scale = None if part.scale is None else part.scale[:, :L]
-                    kernels.head_product(rows, w_uk[h0:h1], out=k, scale=scale)
-                    kernels.head_product(rows, w_uv[h0:h1], out=v, scale=scale)
+                    kernels.head_product(rows, w_uk if whole else w_uk[h0:h1], out=k, scale=scale)
+                    kernels.head_product(rows, w_uv if whole else w_uv[h0:h1], out=v, scale=scale)
                     kernels.prompt_attention(qs, cos, sin, k, v, part, self.softmax_scale, out=os, **kw)
         except torch.OutOfMemoryError:
             return None
