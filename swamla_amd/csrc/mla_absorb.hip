@@ -41,7 +41,8 @@
 // Measured (16 heads, graph-replayed; the kernel before this one, with 16x16
 // MFMAs, a loader wave and 8-byte stores, in brackets): q_abs 36.1 us at 16,384
 // rows [60], 9.8 at 2,048 [12.6]; o 38.9 [45] and 9.2 [9.8]; keys or values of
-// 16,384 latents 29.8 (2.3 TB/s of y), of 8,192 at K = 1024 55 (630 TFLOP/s).
+// 16,384 latents 29.8 alone (2.3 TB/s of y) and 36-37 inside a forward, of 8,192
+// at K = 1024 55 (630 TFLOP/s).
 //
 // LDS: row r at a pitch of a multiple of 256 bytes, its 16-byte chunk c in
 // slot (c & ~15) | ((c ^ r) & 15): the 16 rows of one operand read hit 16

@@ -37,13 +37,14 @@
 // The heaviest query groups (the last ones) are launched first, over all
 // (sequence, head) pairs in turn: with a multiple of 8 pairs each pair's
 // workgroups land on one XCD and stream its keys through one L2.
-// Measured, 16 heads: 385 us at 4 x 4096 tokens from 0 (895 TFLOP/s of its own
-// flops; the latent-space kernels took 650-700, with 1.8 times the flops), 63
-// at 8 x 1001 (537 on the per-row decode kernel at rank 444), 209 at 4 x 2048
-// with 32 heads (650 over an e4m3 cache).  The matrix units are busy 77 % of
-// the cycles, at a clock that drops to 1.4-1.75 GHz under this load: half the
-// VALU instructions (operand addresses kept in registers, no mask away from
-// the diagonal) changed nothing.
+// Measured (kernel-trace medians inside a forward, over runs and boxes), 16
+// heads: 405-411 us at 4 x 4096 tokens from 0 (835-850 TFLOP/s of its own
+// flops; the latent-space kernels took 650-700, with 1.8 times the flops),
+// 63-70 at 8 x 1001 (537 on the per-row decode kernel at rank 444), 227-238 at
+// 4 x 2048 with 32 heads (650 over an e4m3 cache).  The matrix units are busy
+// 77 % of the cycles, at a clock that drops to 1.4-1.75 GHz under this load:
+// half the VALU instructions (operand addresses kept in registers, no mask
+// away from the diagonal) changed nothing.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -420,7 +421,7 @@ __global__ __launch_bounds__(kPrWaves * 64, 2) void mla_prompt_kernel(PromptArgs
 //   O^T[32 x 32 q]: k slot (register r = 4 a + e, half f) is token 8 a + 4 f + e,
 //       the score registers as they are; block i's row m is channel 4 m + i,
 //       so one 16-byte load of a V row serves the four blocks.
-// Measured, 1 x 512 tokens, 16 heads: 32 us against 484 for the per-row VALU
+// Measured, 1 x 512 tokens, 16 heads: 33 us against 484 for the per-row VALU
 // kernel (the longest block's 16 tiles are two per wave: 9 us of MFMAs).
 constexpr int kPfWaves = 8;
 constexpr int kPfQPitch = 196;  // floats per Q row: 49 16-byte chunks, so 16 rows of a read hit distinct banks

@@ -323,7 +323,8 @@ class MLA(nn.Module):
         """``w``, a view of the parameter ``src``, or a copy of it where the
         kernels' 16-byte loads need one (a parameter inside a flat buffer may
         start anywhere; the copy is kept until ``src`` changes)."""
-        if w.data_ptr() % 16 == 0 and w.stride(-1) == 1 and w.stride(-2) % 8 == 0:
+        *_, rs, cs = w.stride()
+        if cs == 1 and rs % 8 == 0 and w.data_ptr() % 16 == 0:
             return w
         return self._derived(name + ".operand", src, lambda: w.clone(memory_format=torch.contiguous_format))
 
@@ -525,7 +526,8 @@ class MLA(nn.Module):
         copy while its grid fits the CUs in one round; past that, or for a K
         or N the kernels do not take, the library GEMM; else mla_linear."""
         n, K = x.shape
-        if x.data_ptr() % 16 != 0 or x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < K:
+        rs, cs = x.stride()
+        if cs != 1 or rs % 8 != 0 or rs < K or x.data_ptr() % 16 != 0:
             x = x.clone(memory_format=torch.contiguous_format)  # rows as the kernels' 16-byte loads need them
         if wp is not None and kernels.packed_ok(n, wp.N, wp.K):
             if self._num_cus is None:
@@ -877,27 +879,26 @@ class MLA(nn.Module):
     def _start_positions(self, B: int, T: int, start_pos, cache: LatentCache, device) -> torch.Tensor:
         """int32 [B] device tensor of per-sequence start positions (checked
         against the cache when given as an int, as mla.py:413 would raise)."""
-        if B > cache.ckv.shape[0]:
-            raise ValueError(f"batch {B} exceeds max_batch_size {cache.ckv.shape[0]}")
+        rows, seq = cache.ckv.shape[:2]
+        if B > rows:
+            raise ValueError(f"batch {B} exceeds max_batch_size {rows}")
         if isinstance(start_pos, torch.Tensor):
             if start_pos.numel() != B:
                 raise ValueError(f"start_pos tensor has {start_pos.numel()} entries for batch {B}")
             if start_pos.device.type == "cpu":  # values known on the host: check them now
                 lo_, hi_ = int(start_pos.min()), int(start_pos.max())
-                if lo_ < 0 or hi_ + T > cache.ckv.shape[1]:
-                    raise ValueError(f"start_pos in [{lo_}, {hi_}] + seqlen {T} is outside max_seq_len "
-                                     f"{cache.ckv.shape[1]}")
+                if lo_ < 0 or hi_ + T > seq:
+                    raise ValueError(f"start_pos in [{lo_}, {hi_}] + seqlen {T} is outside max_seq_len {seq}")
             # device values are checked by the kernels (the module's error flag)
             sp = start_pos.to(device=device, dtype=torch.int32).reshape(-1)
             return sp if sp.is_contiguous() else sp.contiguous()
         start_pos = int(start_pos)
-        if start_pos < 0 or start_pos + T > cache.ckv.shape[1]:
-            raise ValueError(f"start_pos {start_pos} + seqlen {T} exceeds max_seq_len {cache.ckv.shape[1]}")
+        if start_pos < 0 or start_pos + T > seq:
+            raise ValueError(f"start_pos {start_pos} + seqlen {T} exceeds max_seq_len {seq}")
         tab = self._positions
         # a captured call owns what it reads; a cache put in place of the
         # module's own, or moved with it, has no table
-        if (T > 1 or tab is None or tab.shape[0] < cache.ckv.shape[1] or tab.shape[1] < cache.ckv.shape[0]
-                or tab.device != device or self._capturing()):
+        if T > 1 or tab is None or tab.shape != (seq, rows) or tab.device != device or self._capturing():
             return torch.full((B,), start_pos, dtype=torch.int32, device=device)
         return tab[start_pos, :B]
 
