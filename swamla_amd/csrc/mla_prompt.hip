@@ -37,7 +37,7 @@
 // The heaviest query groups (the last ones) are launched first, over all
 // (sequence, head) pairs in turn: with a multiple of 8 pairs each pair's
 // workgroups land on one XCD and stream its keys through one L2.
-// Measured (kernel-trace medians inside a forward, over runs and boxes), 16
+// Measured (kernel-trace medians inside a forward, several runs), 16
 // heads: 405-411 us at 4 x 4096 tokens from 0 (835-850 TFLOP/s of its own
 // flops; the latent-space kernels took 650-700, with 1.8 times the flops),
 // 63-70 at 8 x 1001 (537 on the per-row decode kernel at rank 444), 227-238 at
